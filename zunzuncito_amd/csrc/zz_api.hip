@@ -385,9 +385,10 @@ static int zz_item_slots(int E, int P, int S, int tch) {
 }
 
 // An expert's gate + up weight stream expressed in token columns of the FFN's
-// epilogue work (the dispatch kernel's XCD balance): ~29 for q4_0, where 2.2 MB of
-// weights take as long at HBM speed as 29 columns of 3 VALU operations per weight
-// row and 32-weight block take on the XCD's SIMDs.
+// epilogue work (the dispatch kernel's XCD balance): ~29 for q4_0's 2.2 MB at three VALU
+// operations per weight row, 32-weight block and column, ~44 at the present two. The step
+// does not see the difference (Gemma S = 512 212.0 us at 29, 211.9 at 40, 212.5 at 52,
+// 212.4 at 70; S = 1500 and LFM S = 256 the same within 0.6 %).
 static int zz_weight_cost(const ZzLayout &lay, const zz_moe_desc &d) {
     const double bytes = (double)(lay.gate.fmt == ZZ_FMT_Q80 ? 34 : lay.gate.fmt == ZZ_FMT_TQ2 ? 8.125 : 18) / 32.0 +
                          (double)(lay.up.fmt == ZZ_FMT_Q80 ? 34 : lay.up.fmt == ZZ_FMT_TQ2 ? 8.125 : 18) / 32.0;

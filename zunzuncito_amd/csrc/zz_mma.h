@@ -10,15 +10,16 @@
 //
 // Work unit: (item, tile). An item is one expert with up to 64 of its tokens (the
 // dispatch work list); a tile is 64 weight rows: 4 waves x one 16-row group each.
-// Every wave multiplies its rows by all of the item's tokens (up to 8 MFMA tiles of
+// Every wave multiplies its rows by all of the item's tokens (up to 4 MFMA tiles of
 // 16 tokens), so each weight fragment is loaded and unpacked once per item.
 //   up:   hidden rows 32*rb..+31: waves 0, 1 the gate groups, waves 2, 3 the up
-//         groups; then h = act(g, u) and its per-token q8_0 quantisation
-//         (gemma4.c:642-645, lfm25.c:712-723, maple.c:665-684) in registers;
+//         groups; then, through LDS, h = act(g, u) and its per-token q8_0 quantisation
+//         (gemma4.c:642-645, lfm25.c:712-723, maple.c:665-684);
 //   down: rows 64*rt..+63 of down; the unweighted y[token*K + slot][row] for the combine.
 // The K loop walks the slot table's chunks of 4 blocks. Weights go straight to
-// registers, two chunks ahead: the slot table holds each lane's bytes for a chunk
-// contiguously (zz_common.h). Activations are staged through LDS, one chunk ahead.
+// registers, three chunks ahead: the slot table holds each lane's bytes for a chunk
+// contiguously (zz_common.h). Activations are staged through LDS, requested two chunks
+// ahead (q8_0: one).
 #pragma once
 #include "zz_common.h"
 #include "zz_kernels.h"
@@ -36,16 +37,18 @@ typedef int zz_v4i __attribute__((ext_vector_type(4)));
 
 struct MmStage {
     __attribute__((aligned(16))) int8_t x[MM_TN][MM_XS];
-    float s[4][MM_TN];               // block scales d_x, [block][token]
+    __attribute__((aligned(16))) float s[MM_TN][4];      // block scales d_x, [token][block]
 };
 
 // One wave's weight operand for one chunk (4 blocks, or 2 in a short last chunk).
 //   q4_0: q = the lane's 4 words (k 8qq..8qq+7 of each block, zz_common.h)
 //   q8_0: q, q2 = the lane's 32 bytes
 //   tq2:  q.xy, q.zw = 8 bytes of row r's 64-groups 2c, 2c+1 (bit planes)
-// s0, s1: fp16 scales of rows 4qq..4qq+3, [row][block] (q4_0, q8_0).
+// s: the fp16 scales of the lane's row (q4_0, q8_0): [block] of a full chunk; of a short
+// one the words of rows r & ~1 and r | 1 (an aligned 8-byte load, inside the plane).
 struct MmA {
-    uint4 q, q2, s0, s1;
+    uint4 q, q2;
+    uint2 s;
 };
 
 template <int FMT>
@@ -53,7 +56,7 @@ __device__ __forceinline__ MmA mm_load_a(const uint8_t *E, const ZzTensor &T, co
                                          int l) {
     const int r = l & 15, qq = l >> 4;
     const uint4 z = make_uint4(0, 0, 0, 0);
-    MmA A = {z, z, z, z};
+    MmA A = {z, z, make_uint2(0, 0)};
     if (FMT == ZZ_FMT_TQ2) {
         const int ng = T.I / 64, row = 16 * g + r;
         const uint2 v0 = *(const uint2 *)(E + zz_tq2off(T, row, 2 * c) + (qq & 1) * 8);
@@ -63,19 +66,18 @@ __device__ __forceinline__ MmA mm_load_a(const uint8_t *E, const ZzTensor &T, co
     }
     // Branch-free: the same loads on every path (only addresses are selected), so
     // the compiler's load counters stay exact across the pipelined loops. A short
-    // last chunk (2 blocks) has 8 (q4_0) or 16 (q8_0) bytes per lane and 4 scale
-    // words per lane group; the extra bytes read stay inside the slot (the q plane
-    // is followed by the scale plane) and belong to blocks the loop skips.
+    // last chunk (2 blocks) has 8 (q4_0) or 16 (q8_0) bytes and one scale word per lane;
+    // the extra bytes read stay inside the slot (the q plane is followed by the scale
+    // plane) and belong to blocks the loop skips.
     const bool full = c < W.nfull;
-    const uint32_t qo = zz_walk_qo(W, c), so = zz_walk_so(W, c);    // so: 16-byte aligned
+    const uint32_t qo = zz_walk_qo(W, c), so = zz_walk_so(W, c);
     A.q = ld16(E + qo);
     if (FMT == ZZ_FMT_Q80) A.q2 = ld16(E + (qo + (full ? 16u : 0u)));
-    A.s0 = ld16(E + so);
-    A.s1 = ld16(E + (so + (full ? 16u : 0u)));
+    A.s = *(const uint2 *)(E + (full ? so : so & ~7u));
     return A;
 }
 
-// A fragment of block j (8 signed int8, k = 8qq..8qq+7 of the lane's row)
+// weight operand of block j (8 signed int8, k = 8qq..8qq+7 of the lane's row)
 template <int FMT>
 __device__ __forceinline__ long mm_frag(const MmA &A, int j, int l) {
     if (FMT == ZZ_FMT_Q80) {
@@ -90,76 +92,112 @@ __device__ __forceinline__ long mm_frag(const MmA &A, int j, int l) {
         return (long)((unsigned long)u.x | ((unsigned long)u.y << 32));
     }
     // tq2: block j is half j&1 of group j/2; k 0..15 of a half are bit plane
-    // 2*(j&1), k 16..31 plane 2*(j&1)+1, byte k%16 (tq2.h:46-51)
+    // 2*(j&1), k 16..31 plane 2*(j&1)+1, byte k%16 (tq2.h:46-51). mm_chunk flips bit 0 of
+    // every code c: c ^ 1 is 1 - c in two bits of two's complement for every c (0..3), and
+    // moved to the top of its byte it is the int8 -64 (c - 1), two operations per four
+    // weights (forming c - 1 itself took four).
     const uint2 v = j < 2 ? make_uint2(A.q.x, A.q.y) : make_uint2(A.q.z, A.q.w);
-    const unsigned sh = 2 * (2 * (j & 1) + ((l >> 4) >> 1));
-    unsigned x = (v.x >> sh) & 0x03030303u, y = (v.y >> sh) & 0x03030303u;
-    x = (x + 0x7F7F7F7Fu) ^ 0x80808080u;          // bytewise c - 1
-    y = (y + 0x7F7F7F7Fu) ^ 0x80808080u;
-    return (long)((unsigned long)x | ((unsigned long)y << 32));
+    const unsigned sh = 6 - 4 * (j & 1) - 2 * (l >> 5);
+    return (long)((unsigned long)((v.x << sh) & 0xC0C0C0C0u) | ((unsigned long)((v.y << sh) & 0xC0C0C0C0u) << 32));
 }
 
-// d_w of row 4qq+i, block j of the chunk, as fp16: halfword i*cbs + j of s0|s1
-// (i, j and the chunk size compile-time, so this is a register and a half select).
+// d_w of the lane's row r, block j of the chunk (MmA::s)
 template <bool FULL>
-__device__ __forceinline__ _Float16 mm_dwh(const uint4 &s0, const uint4 &s1, int j, int i) {
-    const int h = FULL ? 4 * i + j : 2 * i + j, w = h >> 1;
-    const unsigned u = w == 0 ? s0.x : w == 1 ? s0.y : w == 2 ? s0.z : w == 3 ? s0.w
-                     : w == 4 ? s1.x : w == 5 ? s1.y : w == 6 ? s1.z : s1.w;
-    return __builtin_bit_cast(_Float16, (unsigned short)((h & 1) ? u >> 16 : u & 0xffff));
+__device__ __forceinline__ float mm_dw(uint2 s, int j, int r) {
+    const unsigned w = FULL ? (j < 2 ? s.x : s.y) : (s.x ^ ((s.x ^ s.y) & -(unsigned)(r & 1)));
+    return (float)__builtin_bit_cast(_Float16, (unsigned short)((j & 1) ? w >> 16 : w & 0xffff));
 }
 
-// One chunk: acc[t][i] += d_w * d_x * <w, x> for row 4qq+i of the wave's row group
-// and token 16t + l%16, over the chunk's 4 (FULL) or 2 blocks. X(t, j) is the 8-byte
-// B operand of token tile t, block j; SX(t, j) that token's d_x.
-// Per product: d_w * d_x (a multiply by the block's d_w, converted once per block),
-// the int32 conversion, the accumulating FMA.
-// DF(j, r): called with block j's int32 results before their scaling (diagnostics
-// builds store them; the timed build passes a hook that does nothing).
-template <int FMT, int NT, bool FULL, typename XF, typename SF, typename DF>
-__device__ __forceinline__ void mm_chunk(const MmA &A, int l, float (&acc)[NT][4], XF X, SF SX, DF dbg) {
-    const zz_v4i zero = {0, 0, 0, 0};
+// The matrix cores add the block's dot to an integer C operand. With C the bits of the
+// float MM_M = 1.5 * 2^23 the result's bits are the float MM_M + dot, exactly: every dot
+// here is below 2^20 in magnitude (q4_0 16 * 8 * 127 * 32, q8_0 127 * 127 * 32), and from
+// 2^23 to 2^24 a float's unit is 1. fma(MM_M + dot, d_w, -MM_M * d_w) then is d_w * dot
+// rounded once: -MM_M * d_w is exact (3 * 2^22 times fp16's 11 bits), so the product needs
+// no integer conversion. tq2 has no block scale and keeps the conversion.
+#define MM_MBITS 0x4B400000
+#define MM_M 12582912.0f
+
+// acc[i] += p[i] * (lane J0 + i's value of sx, in each row of 16 lanes). The compiler
+// leaves the broadcast a move of its own (a third operation per output), so the
+// multiply-add with the DPP operand is written out. s_nop 1: the two wait states a DPP
+// read needs after a VALU write of its source.
+#define MM_FD(A, P, X, J) "v_fmac_f32_dpp %" #A ", %" #X ", %" #P " row_newbcast:" #J " row_mask:0xf bank_mask:0xf\n\t"
+#define MM_FD4(J0, J1, J2, J3)                                                                        \
+    asm("s_nop 1\n\t" MM_FD(0, 4, 8, J0) MM_FD(1, 5, 8, J1) MM_FD(2, 6, 8, J2) MM_FD(3, 7, 8, J3)     \
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])                                      \
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(sx))
+template <int T>
+__device__ __forceinline__ void mm_fmac4(float (&acc)[4], const float (&p)[4], float sx) {
+    if constexpr (T == 0) MM_FD4(0, 1, 2, 3);
+    else if constexpr (T == 1) MM_FD4(4, 5, 6, 7);
+    else if constexpr (T == 2) MM_FD4(8, 9, 10, 11);
+    else MM_FD4(12, 13, 14, 15);
+}
+#undef MM_FD4
+#undef MM_FD
+
+// acc[t][i] += (d_w * dot) * d_x over the tiles of one block. Lane l holds weight row
+// l%16 of its group, VGPR i of tile t token 16t + 4(l/16) + i; lane 16qq + n of sx holds
+// the d_x of token 16(n/4) + 4qq + n%4, so that token's d_x reaches the lanes of its
+// quarter as the DPP row broadcast of lane 4t + i, folded into the multiply-add.
+template <int FMT, int NT, int t = 0>
+__device__ __forceinline__ void mm_epi(float (&acc)[NT][4], const zz_v4i (&r)[NT], float dw, float nm, float sx) {
+    if constexpr (t < NT) {
+        float p[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            p[i] = FMT == ZZ_FMT_TQ2 ? (float)r[t][i] : fmaf(__int_as_float(r[t][i]), dw, nm);
+        mm_fmac4<t>(acc[t], p, sx);
+        mm_epi<FMT, NT, t + 1>(acc, r, dw, nm, sx);
+    }
+}
+
+// One chunk: acc[t][i] += d_w * d_x * <w, x> for row l%16 of the wave's row group and
+// token 16t + 4(l/16) + i, over the chunk's 4 (FULL) or 2 blocks. X(t, j) is the 8-byte
+// activation operand of token tile t, block j (lane l: token 16t + l%16); sx[j] the lane's
+// d_x of block j (mm_epi). The activations are the matrix cores' A rows and the weights
+// their B columns: a lane then holds ONE weight row, whose d_w costs one conversion and one
+// product a block. Bound by VALU issue from three tiles on: with the weights as A rows a
+// lane held four rows (four of each a block) and an output took three operations (d_w * d_x,
+// the integer conversion, the multiply-add) where two do now, 14.0 VALU operations per
+// matrix-core instruction against 10.7 over the whole up kernel. Gemma-4 layer, S = 512,
+// Zipf routing: ffn_up 94.8 -> 86.1 us, ffn_down 61.1 -> 58.2; LFM S = 256 61.0 -> 51.5 and
+// 44.2 -> 38.9; Maple (tq2) S = 512 95.7 -> 86.4 and 59.5 -> 55.6 (HIP events).
+// DF(j, r): called with block j's int32 results, MM_MBITS added to each except tq2's
+// (diagnostics builds store them; the timed build passes a hook that does nothing).
+template <int FMT, int NT, bool FULL, typename XF, typename DF>
+__device__ __forceinline__ void mm_chunk(MmA A, int l, float (&acc)[NT][4], XF X, const float4 &sx4, DF dbg) {
+    constexpr int C0 = FMT == ZZ_FMT_TQ2 ? 0 : MM_MBITS;
+    const zz_v4i c0 = {C0, C0, C0, C0};
+    const float sx[4] = {sx4.x, sx4.y, sx4.z, sx4.w};
+    if (FMT == ZZ_FMT_TQ2)                       // here, not at the load: that would wait for it
+        A.q = make_uint4(A.q.x ^ 0x55555555u, A.q.y ^ 0x55555555u, A.q.z ^ 0x55555555u, A.q.w ^ 0x55555555u);
 #pragma unroll
     for (int j = 0; j < (FULL ? 4 : 2); j++) {
-        const long fa = mm_frag<FMT>(A, j, l);
+        const long fw = mm_frag<FMT>(A, j, l);
         long B[NT];
-        float sx[NT];
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-            B[t] = X(t, j);
-            sx[t] = SX(t, j);
-        }
+        for (int t = 0; t < NT; t++) B[t] = X(t, j);
         // all tiles' products first, into distinct registers, so that each epilogue
         // finds its matrix-core result ready instead of waiting on it
         zz_v4i r[NT];
 #pragma unroll
-        for (int t = 0; t < NT; t++) r[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fa, B[t], zero, 0, 0, 0);
+        for (int t = 0; t < NT; t++) r[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(B[t], fw, c0, 0, 0, 0);
         dbg(j, r);
-        // the 4 rows' d_w as f32 once per block, for every tile: the product d_w * d_x
-        // is then a v_mul_f32, which ran the up kernel 3 % faster than the fused
-        // mixed-precision form (v_fma_mix_f32) the compiler otherwise picks; the empty
-        // asm keeps it from folding them back together. tq2 has no block scale (its
-        // alpha is per row), and no asm: pinned, the constant 1 cost four moves a block.
-        float dwf[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+        float dw = 1.0f, nm = 0.0f;
         if constexpr (FMT != ZZ_FMT_TQ2) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                dwf[i] = (float)mm_dwh<FULL>(A.s0, A.s1, j, i);
-                asm volatile("" : "+v"(dwf[i]));
-            }
+            // the empty asm keeps the conversion from being folded into each product as
+            // the slower mixed-precision v_fma_mix_f32
+            dw = mm_dw<FULL>(A.s, j, l);
+            asm("" : "+v"(dw));
+            nm = dw * -MM_M;
         }
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float s = FMT == ZZ_FMT_TQ2 ? sx[t] : dwf[i] * sx[t];
-                acc[t][i] = fmaf(s, (float)r[t][i], acc[t][i]);
-            }
-        }
-        // three or four tiles: one block at a time (the next block's LDS reads hoisted
-        // over this one would hold NT more operand registers); one or two tiles leave
-        // the scheduler free to overlap them (0.5 us off each FFN kernel at S = 512)
-        if (NT >= 3) __builtin_amdgcn_sched_barrier(0);
+        mm_epi<FMT, NT>(acc, r, dw, nm, sx[j]);
+        // three or four tiles (q8_0 two): one block at a time (the next block's LDS reads
+        // hoisted over this one would hold NT more operand registers: q8_0 spilled 28);
+        // fewer leave the scheduler free to overlap them (0.5 us off each FFN kernel at
+        // S = 512)
+        if (NT >= 3 || (NT == 2 && FMT == ZZ_FMT_Q80)) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -206,7 +244,7 @@ __device__ __forceinline__ void mm_store_x(const MmX &x, MmStage &st) {
 #pragma unroll
     for (int k = 0; k < MM_SP; k++) {
         const int i = tid + 256 * k;
-        st.s[i / MM_TN][i % MM_TN] = x.s[k];
+        st.s[i >> 2][i & 3] = x.s[k];
     }
 }
 
@@ -216,9 +254,8 @@ __device__ __forceinline__ void mm_store_x(const MmX &x, MmStage &st) {
 // rings of full chunks with every load unconditional (clamped past the end); the
 // remaining chunks (fewer than RING + 1, the short one last) run in a tail.
 //
-// Large items: activations one chunk ahead through the two LDS stages, one
-// workgroup barrier per chunk.
-template <int FMT, int NT, int RING, typename DF>
+// Large items: activations through the two LDS stages, one workgroup barrier per chunk.
+template <int FMT, int NT, int RING, int XD, typename DF>
 __device__ __forceinline__ void mm_kloop(const uint8_t *E, const ZzTensor &T, int g, const MmSrc &src,
                                          MmStage (&st)[2], float (&acc)[NT][4], DF dbgc) {
     const int l = threadIdx.x & 63, nb = T.I / ZZ_BLK, nch = (nb + 3) / 4, nfull = nb / 4;
@@ -227,50 +264,57 @@ __device__ __forceinline__ void mm_kloop(const uint8_t *E, const ZzTensor &T, in
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[t][i] = 0.0f;
     constexpr int KP = (NT + 1) / 2 < MM_XP ? (NT + 1) / 2 : MM_XP;
-    const ZzWalk W = zz_walk(T, g, l, 4 * (l >> 4));
+    const ZzWalk W = zz_walk(T, g, l, l & 15);
     MmA r[RING];
+    // the activations of chunk c are requested XD (1 or 2) steps ahead, into
+    // xr[c % XD], and stored to stage c % 2 at the end of step c - 1
+    static_assert(XD == 1 || RING % 2 == 0, "xr's index is static in the unrolled ring");
+    MmX xr[XD];
+    auto load_x = [&](int c, MmX &x) {
+        const int c1 = min(c, nch - 1);
+        mm_load_x<KP>(src, c1, min(4, nb - 4 * c1), x);
+    };
+    load_x(0, xr[0]);
 #pragma unroll
     for (int i = 0; i < RING - 1; i++) r[i] = mm_load_a<FMT>(E, T, W, g, min(i, nch - 1), l);
-    MmX xr;
-    mm_load_x<KP>(src, 0, min(4, nb), xr);
-    mm_store_x<KP>(xr, st[0]);
-    // x of chunk c + 1 is requested before the weight prefetch: the wait for it at
-    // the end of the step (loads complete in order) then leaves the prefetch in flight
-    auto load_x = [&](int c) {
-        const int c1 = min(c + 1, nch - 1);
-        mm_load_x<KP>(src, c1, min(4, nb - 4 * c1), xr);
-    };
-    auto step = [&](int c, const MmA &A, auto full) {
+    if (XD == 2) load_x(1, xr[XD - 1]);
+    mm_store_x<KP>(xr[0], st[0]);
+    auto step = [&](int c, const MmA &A, const MmX &x1, auto full) {
         __syncthreads();                         // stage c%2 complete; stage (c+1)%2 free
         const MmStage &S = st[c & 1];
+        const float4 sx = *(const float4 *)S.s[16 * ((l & 15) >> 2) + 4 * (l >> 4) + (l & 3)];
         mm_chunk<FMT, NT, decltype(full)::value>(
             A, l, acc, [&](int t, int j) { return *(const long *)&S.x[16 * t + (l & 15)][j * ZZ_BLK + 8 * (l >> 4)]; },
-            [&](int t, int j) { return S.s[j][16 * t + (l & 15)]; },
-            [&](int j, const zz_v4i (&rr)[NT]) { dbgc(c, j, rr); });
-        mm_store_x<KP>(xr, st[(c + 1) & 1]);     // the last step refills the free stage: harmless
+            sx, [&](int j, const zz_v4i (&rr)[NT]) { dbgc(c, j, rr); });
+        mm_store_x<KP>(x1, st[(c + 1) & 1]);     // the last step refills the free stage: harmless
     };
     int c0 = 0;
     for (; c0 + RING <= nfull; c0 += RING) {
 #pragma unroll
         for (int u = 0; u < RING; u++) {
-            load_x(c0 + u);
+            load_x(c0 + u + XD, xr[u % XD]);
             r[(u + RING - 1) % RING] = mm_load_a<FMT>(E, T, W, g, min(c0 + u + RING - 1, nch - 1), l);
-            step(c0 + u, r[u], std::true_type());
+            step(c0 + u, r[u], xr[(u + 1) % XD], std::true_type());
         }
     }
 #pragma unroll
     for (int u = 0; u < RING; u++) {
         const int c = c0 + u;
         if (c < nch) {
-            load_x(c);
+            load_x(c + XD, xr[u % XD]);
             if (u == RING - 1) r[u] = mm_load_a<FMT>(E, T, W, g, c, l);
-            if (c < nfull) step(c, r[u], std::true_type());
-            else step(c, r[u], std::false_type());
+            if (c < nfull) step(c, r[u], xr[(u + 1) % XD], std::true_type());
+            else step(c, r[u], xr[(u + 1) % XD], std::false_type());
         }
     }
 }
 
-#define MM_RING(NT) ((NT) <= 2 ? 4 : 3)
+// Weight ring and activation depth. With one weight row a lane its chunk takes 6 (q4_0) or
+// 10 (q8_0) registers instead of 12 and 16, which pays for four sets at every tile count
+// (three before, from three tiles on) and, but for q8_0, for activations two chunks ahead:
+// Maple S = 512 ffn_up 90.1 us with three sets and one chunk ahead, 85.7 with these.
+#define MM_RING 4
+#define MM_XD(FMT) ((FMT) == ZZ_FMT_Q80 ? 1 : 2)
 
 // ------------------------------------------------------------------ tiny items
 // Items of <= 4 tokens (the long tail of experts under skewed routing) would fill a
@@ -318,6 +362,16 @@ __device__ __forceinline__ void mm4_stage(Mm4Stage &st, RF row, SF srow, int K) 
         st.s[t * MM4_SS(K) + b] = srow(t)[b];
     }
     __syncthreads();
+}
+
+// d_w of row 4qq+i, block j of the chunk, as fp16: halfword i*cbs + j of s0|s1
+// (i, j and the chunk size compile-time, so this is a register and a half select).
+template <bool FULL>
+__device__ __forceinline__ _Float16 mm_dwh(const uint4 &s0, const uint4 &s1, int j, int i) {
+    const int h = FULL ? 4 * i + j : 2 * i + j, w = h >> 1;
+    const unsigned u = w == 0 ? s0.x : w == 1 ? s0.y : w == 2 ? s0.z : w == 3 ? s0.w
+                     : w == 4 ? s1.x : w == 5 ? s1.y : w == 6 ? s1.z : s1.w;
+    return __builtin_bit_cast(_Float16, (unsigned short)((h & 1) ? u >> 16 : u & 0xffff));
 }
 
 // A lane's chunk: its row's four pieces (q4_0 16 bytes each, q8_0 32) and the fp16

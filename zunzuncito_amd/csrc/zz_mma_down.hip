@@ -30,9 +30,9 @@ __device__ __forceinline__ void mm_down_body(const ZzFfnArgs &a, const ZzItem &i
     }
 #pragma unroll
     for (int k = 0; k < MM_SP; k++) {
-        const int i = tid + 256 * k, t = i % MM_TN;
+        const int i = tid + 256 * k, t = i >> 2;
         src.srow[k] = (uint32_t)(item.p0 + min(t, n - 1)) * (uint32_t)(4 * nb);
-        src.kb[k] = i / MM_TN;
+        src.kb[k] = i & 3;
     }
 
     auto dbgc = [&](int c, int j, const zz_v4i (&rr)[NT]) {
@@ -40,30 +40,26 @@ __device__ __forceinline__ void mm_down_body(const ZzFfnArgs &a, const ZzItem &i
 #pragma unroll
             for (int t = 0; t < NT; t++)
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (16 * t + (l & 15) < n)
-                        mm_dbg_dn(a, item.p0 + 16 * t + (l & 15), 16 * g + 4 * qq + i, 4 * c + j, rr[t][i]);
+                for (int i = 0; i < 4; i++) {
+                    const int tk = 16 * t + 4 * qq + i;
+                    if (tk < n)
+                        mm_dbg_dn(a, item.p0 + tk, 16 * g + (l & 15), 4 * c + j,
+                                  FMT == ZZ_FMT_TQ2 ? -rr[t][i] / 64 : rr[t][i] - MM_MBITS);
+                }
         }
     };
     float acc[NT][4];
-    const int row0 = 16 * g + 4 * qq;
-    float al[4] = {1.0f, 1.0f, 1.0f, 1.0f};     // tq2's row alpha: read now, used at the end
-    if (FMT == ZZ_FMT_TQ2)
+    const int row = 16 * g + (l & 15);
+    // q4_0: the 16*(q - 8) weights; tq2: the row alpha, read now, used at the end
+    const float f = FMT == ZZ_FMT_Q40 ? 0.0625f : FMT == ZZ_FMT_TQ2 ? ((const float *)(E + T.off_s))[row] * -0.015625f : 1.0f;
+    mm_kloop<FMT, NT, MM_RING, MM_XD(FMT)>(E, T, g, src, sm.st, acc, dbgc);
 #pragma unroll
-        for (int i = 0; i < 4; i++) al[i] = ((const float *)(E + T.off_s))[row0 + i];
-    mm_kloop<FMT, NT, MM_RING(NT)>(E, T, g, src, sm.st, acc, dbgc);
-    if (FMT == ZZ_FMT_Q40)                       // the 16*(q - 8) weights
+    for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[t][i] *= 0.0625f;
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const int tk = 16 * t + (l & 15);
-        if (tk < n)
-            *(float4 *)(a.y + (size_t)yrow[tk] * a.D + row0) =
-                make_float4(acc[t][0] * al[0], acc[t][1] * al[1], acc[t][2] * al[2], acc[t][3] * al[3]);
-    }
+        for (int i = 0; i < 4; i++) {
+            const int tk = 16 * t + 4 * qq + i;
+            if (tk < n) a.y[(size_t)yrow[tk] * a.D + row] = acc[t][i] * f;
+        }
 }
 
 // Tiny items (<= 4 NS tokens), down: rows 64rt + l, the unweighted y of each token.

@@ -7,11 +7,7 @@
 union MmUpShared {
     MmStage st[2];
     Mm4Shared t4;
-    struct {
-        float u[32][MM_TN + 1];              // up values, [hidden row][token]
-        float amax[2][MM_TN];
-        int qsum[2][MM_TN];
-    } e;
+    float gu[2][MM_TN][ZZ_BLK + 4];          // gate and up values, [token][hidden row]
 };
 
 // GF, UF: the gate and up formats (gate and up are both tq2 or neither)
@@ -35,97 +31,60 @@ __device__ __forceinline__ void mm_up_body(const ZzFfnArgs &a, const ZzItem &ite
     }
 #pragma unroll
     for (int k = 0; k < MM_SP; k++) {
-        const int i = tid + 256 * k, t = i % MM_TN;
+        const int i = tid + 256 * k, t = i >> 2;
         src.srow[k] = (uint32_t)tok[t] * (uint32_t)(4 * nb);
-        src.kb[k] = i / MM_TN;
+        src.kb[k] = i & 3;
     }
 
     // gate and up may differ in format (q4_0 / q8_0); each wave runs its tensor's loop
     // (the same number of chunks and barriers either way)
-    // lane l, tile t, VGPR i: row 16g + 4qq + i of the wave's tensor, token 16t + l%16
+    // lane l, tile t, VGPR i: row 16g + l%16 of the wave's tensor, token 16t + 4qq + i
     auto dbgc = [&](int c, int j, const zz_v4i (&rr)[NT]) {
         if constexpr (DBG) {
 #pragma unroll
             for (int t = 0; t < NT; t++)
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (16 * t + (l & 15) < n)
-                        mm_dbg_up(a, item.p0 + 16 * t + (l & 15), w < 2 ? 0 : 1, 16 * g + 4 * qq + i, 4 * c + j, rr[t][i]);
+                for (int i = 0; i < 4; i++) {
+                    const int tk = 16 * t + 4 * qq + i;
+                    if (tk < n)
+                        mm_dbg_up(a, item.p0 + tk, w < 2 ? 0 : 1, 16 * g + (l & 15), 4 * c + j,
+                                  GF == ZZ_FMT_TQ2 ? -rr[t][i] / 64 : rr[t][i] - MM_MBITS);
+                }
         }
     };
     float acc[NT][4];
-    float alr[4] = {1.0f, 1.0f, 1.0f, 1.0f};     // tq2.h:154, alpha of the row: read now,
-    if (GF == ZZ_FMT_TQ2)                        // used after the K loop
-#pragma unroll
-        for (int i = 0; i < 4; i++) alr[i] = ((const float *)(E + T.off_s))[16 * g + 4 * qq + i];
-    if (GF == UF || w < 2) mm_kloop<GF, NT, MM_RING(NT)>(E, T, g, src, sm.st, acc, dbgc);
-    else mm_kloop<UF, NT, MM_RING(NT)>(E, T, g, src, sm.st, acc, dbgc);
-    if ((w < 2 ? GF : UF) == ZZ_FMT_Q40)         // the 16*(q - 8) weights
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[t][i] *= 0.0625f;
-    if (GF == ZZ_FMT_TQ2) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int t = 0; t < NT; t++) acc[t][i] *= alr[i];
-    }
+    float f = 1.0f;                              // tq2.h:154, alpha of the row: read now,
+    if (GF == ZZ_FMT_TQ2) f = ((const float *)(E + T.off_s))[16 * g + (l & 15)] * -0.015625f;   // used after the K loop
+    if (GF == UF || w < 2) mm_kloop<GF, NT, MM_RING, MM_XD(GF)>(E, T, g, src, sm.st, acc, dbgc);
+    else mm_kloop<UF, NT, MM_RING, MM_XD(UF)>(E, T, g, src, sm.st, acc, dbgc);
+    if ((w < 2 ? GF : UF) == ZZ_FMT_Q40) f = 0.0625f;     // the 16*(q - 8) weights
     __syncthreads();                             // the stages are done with
-    if (w >= 2) {
 #pragma unroll
-        for (int t = 0; t < NT; t++)
+    for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) sm.e.u[16 * (w & 1) + 4 * qq + i][16 * t + (l & 15)] = acc[t][i];
-    }
+        for (int i = 0; i < 4; i++) sm.gu[w >> 1][16 * t + 4 * qq + i][16 * (w & 1) + (l & 15)] = acc[t][i] * f;
     __syncthreads();
-    // waves 0, 1: h = act(g, u) for hidden rows 16w + 4qq + i, then the q8_0
-    // quantisation of each token's 32-row block (q40.h:124-138)
-    float amx[NT];
-    if (w < 2) {
+    // h = act(g, u) and each token's q8_0 block (q40.h:124-138), 8 lanes of 4 hidden rows
+    // per token
+    const int nbM = a.MI / ZZ_BLK, m = tid & 7;
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-            float m = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float h = zz_act(a.act, acc[t][i], sm.e.u[16 * w + 4 * qq + i][16 * t + (l & 15)], a.clamp);
-                acc[t][i] = h;
-                m = fmaxf(m, fabsf(h));
-            }
-            m = zz_rows_max(m);
-            amx[t] = m;
-            if (qq == 0) sm.e.amax[w][16 * t + l] = m;
-        }
-    }
-    __syncthreads();
-    if (w < 2) {
-        const int nbM = a.MI / ZZ_BLK;
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const int tk = 16 * t + (l & 15);
-            const float amax = fmaxf(amx[t], sm.e.amax[w ^ 1][tk]);
-            const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
-            unsigned pk = 0;
-            int s = 0;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float f = rintf(acc[t][i] * id);
-                f = fminf(fmaxf(f, -127.0f), 127.0f);
-                const int qi = (int)f;
-                s += qi;
-                pk |= (unsigned)(qi & 0xff) << (8 * i);
-            }
-            s = zz_rows_sum(s);
-            if (qq == 0) sm.e.qsum[w][tk] = s;
-            if (tk < n) {
-                const size_t p = (size_t)item.p0 + tk;
-                *(unsigned *)(a.hq + p * a.MI + rb * ZZ_BLK + 16 * w + 4 * qq) = pk;
-                if (w == 0 && qq == 0) a.hs[p * nbM + rb] = d;
+    for (int k = 0; k < (NT + 1) / 2; k++) {
+        const int tk = (tid >> 3) + 32 * k;
+        const float4 gv = *(const float4 *)&sm.gu[0][tk][4 * m], uv = *(const float4 *)&sm.gu[1][tk][4 * m];
+        const float4 h = make_float4(zz_act(a.act, gv.x, uv.x, a.clamp), zz_act(a.act, gv.y, uv.y, a.clamp),
+                                     zz_act(a.act, gv.z, uv.z, a.clamp), zz_act(a.act, gv.w, uv.w, a.clamp));
+        float d;
+        int qs;
+        const unsigned pk = zz_quant8(h, &d, &qs);
+        if (tk < n) {
+            const size_t p = (size_t)item.p0 + tk;
+            *(unsigned *)(a.hq + p * a.MI + rb * ZZ_BLK + 4 * m) = pk;
+            if (m == 0) {
+                a.hs[p * nbM + rb] = d;
+                a.hsum[p * nbM + rb] = qs;
             }
         }
     }
-    __syncthreads();
-    if (tid < n) a.hsum[((size_t)item.p0 + tid) * (a.MI / ZZ_BLK) + rb] = sm.e.qsum[0][tid] + sm.e.qsum[1][tid];
 }
 
 // Tiny items (<= 4 NS tokens): lanes 0..31 own gate rows 32rb.., lanes 32..63 the up
