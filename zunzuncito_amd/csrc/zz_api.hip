@@ -542,7 +542,8 @@ struct ChunkArgs {
 // zz_moe_dots: while it runs, the FFN kernels also store their per-block int32 dots
 static int32_t *g_dbg_up = nullptr, *g_dbg_dn = nullptr;
 
-static ChunkArgs chunk_args(Layer *L, Workspace &w, const float *d_in, int S) {
+// d_eidx, d_ewt: where the caller wants this chunk's routing (device [S, K]), or null
+static ChunkArgs chunk_args(Layer *L, Workspace &w, const float *d_in, int S, int *d_eidx, float *d_ewt) {
     const zz_moe_desc &d = L->d;
     ChunkArgs c;
     memset(&c, 0, sizeof c);
@@ -568,6 +569,7 @@ static ChunkArgs chunk_args(Layer *L, Workspace &w, const float *d_in, int S) {
     ta.routed_scaling = d.routed_scaling; ta.cen = w.cen; ta.bnd = w.bnd; ta.router = L->router;
     ta.xn = w.xn; ta.bias = d.use_bias ? L->bias : nullptr; ta.pes = L->pes; ta.eidx = w.eidx;
     ta.ewt = w.ewt; ta.topv = w.topv; ta.diag = g_diag;
+    ta.eidx_out = d_eidx; ta.ewt_out = d_ewt;
 
     // decode-sized batches take the GEMV path; larger ones the matrix cores, on
     // work items of up to ZZ_MMA_TOKENS tokens of one expert
@@ -590,9 +592,10 @@ static ChunkArgs chunk_args(Layer *L, Workspace &w, const float *d_in, int S) {
     return c;
 }
 
-static int run_chunk(Layer *L, Workspace &w, const float *d_in, float *d_out, int S, hipStream_t st) {
+static int run_chunk(Layer *L, Workspace &w, const float *d_in, float *d_out, int S, int *d_eidx, float *d_ewt,
+                     hipStream_t st) {
     const zz_moe_desc &d = L->d;
-    ChunkArgs c = chunk_args(L, w, d_in, S);
+    ChunkArgs c = chunk_args(L, w, d_in, S, d_eidx, d_ewt);
 
     if (c.dec) {
         ZzDecRouteArgs ra;
@@ -664,7 +667,7 @@ int zz_block_decode(int moe_id, int dense_id, float *d_H, float *d_h1, float *d_
     if (L->n_present != d.E || N->n_present != dn.E) ZZ_FAIL("block: experts not uploaded");
     if (!ensure_ws(L, S) || !ensure_ws(N, S)) return 0;
     Workspace &w = L->ws, &wn = N->ws;
-    ChunkArgs c = chunk_args(L, w, d_H, S), cn = chunk_args(N, wn, d_H, S);
+    ChunkArgs c = chunk_args(L, w, d_H, S, d_eidx, d_ewt), cn = chunk_args(N, wn, d_H, S, nullptr, nullptr);
 
     ZzDecRouteArgs ra;
     memset(&ra, 0, sizeof ra);
@@ -692,8 +695,6 @@ int zz_block_decode(int moe_id, int dense_id, float *d_H, float *d_h1, float *d_
     } else if (!(ProfScope(ZZ_K_COMBINE, st), zz_launch_dec_final(fa, S, st))) {
         ZZ_FAIL("block: final launch failed");
     }
-    if (d_eidx) ZZ_CHECK(hipMemcpyAsync(d_eidx, w.eidx, sizeof(int) * S * d.K, hipMemcpyDeviceToDevice, st));
-    if (d_ewt) ZZ_CHECK(hipMemcpyAsync(d_ewt, w.ewt, sizeof(float) * S * d.K, hipMemcpyDeviceToDevice, st));
     L->last_S = N->last_S = S;                  // both layers' hidden rows by flat pair
     L->last_dec = N->last_dec = true;
     return 1;
@@ -705,9 +706,12 @@ static int run_chunks(Layer *L, Workspace &w, int CH, const float *d_in, float *
     const zz_moe_desc &d = L->d;
     for (int s0 = 0; s0 < S; s0 += CH) {
         int n = S - s0 < CH ? S - s0 : CH;
-        if (!run_chunk(L, w, d_in + (size_t)s0 * d.D, d_out + (size_t)s0 * d.D, n, st)) return 0;
-        if (d_eidx) ZZ_CHECK(hipMemcpyAsync(d_eidx + (size_t)s0 * d.K, w.eidx, sizeof(int) * n * d.K, hipMemcpyDeviceToDevice, st));
-        if (d_ewt) ZZ_CHECK(hipMemcpyAsync(d_ewt + (size_t)s0 * d.K, w.ewt, sizeof(float) * n * d.K, hipMemcpyDeviceToDevice, st));
+        int *ei = d_eidx ? d_eidx + (size_t)s0 * d.K : nullptr;
+        float *ew = d_ewt ? d_ewt + (size_t)s0 * d.K : nullptr;
+        if (!run_chunk(L, w, d_in + (size_t)s0 * d.D, d_out + (size_t)s0 * d.D, n, ei, ew, st)) return 0;
+        if (d.gating != ZZ_GATE_DENSE) continue;    // the top-k stored the caller's routing
+        if (ei) ZZ_CHECK(hipMemcpyAsync(ei, w.eidx, sizeof(int) * n * d.K, hipMemcpyDeviceToDevice, st));
+        if (ew) ZZ_CHECK(hipMemcpyAsync(ew, w.ewt, sizeof(float) * n * d.K, hipMemcpyDeviceToDevice, st));
     }
     return 1;
 }
@@ -774,7 +778,7 @@ static int forward_host(Layer *L, const float *in, float *out, int S, int *eidx,
     for (int s0 = 0; s0 < S; s0 += CH) {
         int n = S - s0 < CH ? S - s0 : CH;
         ZZ_CHECK(hipMemcpyAsync(w.in, in + (size_t)s0 * d.D, sizeof(float) * n * d.D, hipMemcpyHostToDevice, g_stream));
-        if (!run_chunk(L, w, w.in, w.out, n, g_stream)) return 0;
+        if (!run_chunk(L, w, w.in, w.out, n, nullptr, nullptr, g_stream)) return 0;
         ZZ_CHECK(hipMemcpyAsync(o.data() + (size_t)s0 * d.D, w.out, sizeof(float) * n * d.D, hipMemcpyDeviceToHost, g_stream));
         ZZ_CHECK(hipMemcpyAsync(ix.data() + (size_t)s0 * d.K, w.eidx, sizeof(int) * n * d.K, hipMemcpyDeviceToHost, g_stream));
         ZZ_CHECK(hipMemcpyAsync(wt.data() + (size_t)s0 * d.K, w.ewt, sizeof(float) * n * d.K, hipMemcpyDeviceToHost, g_stream));
@@ -834,7 +838,7 @@ extern "C" int zz_moe_forward_begin(int id, const float *in, int S) {
     if (L->n_present != d.E) ZZ_FAIL("forward: %d of %d experts uploaded", L->n_present, d.E);
     if (!ensure_ws(L, S)) return 0;
     ZZ_CHECK(hipMemcpyAsync(L->ws.in, in, sizeof(float) * S * d.D, hipMemcpyHostToDevice, g_stream));
-    if (!run_chunk(L, L->ws, L->ws.in, L->ws.out, S, g_stream)) return 0;
+    if (!run_chunk(L, L->ws, L->ws.in, L->ws.out, S, nullptr, nullptr, g_stream)) return 0;
     L->pending_S = S;
     return 1;
 }

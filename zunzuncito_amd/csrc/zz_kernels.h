@@ -41,6 +41,8 @@ struct ZzTopkArgs {
     int *eidx;                  // [S, K]
     float *ewt;                 // [S, K]
     float *topv;                // [S, K] selected scores (debug), or null
+    int *eidx_out;              // the caller's copies of eidx and ewt, or null
+    float *ewt_out;
     unsigned *diag;
 };
 

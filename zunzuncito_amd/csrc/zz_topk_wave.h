@@ -105,7 +105,9 @@ __device__ float zz_gemma_chain(const float *w, const float *xn, int D, const fl
 
 // Gate weights of a selected set (the header's idx / topv): lane l < K holds slot l's
 // centre cj and scale pj. Per slot in parallel, their sum serially in slot order as the
-// reference adds them, then each slot's normalisation. write: store eidx, ewt, topv.
+// reference adds them, then each slot's normalisation. write: store eidx, ewt, topv, and
+// the caller's copies of the first two: two lanes' stores here instead of two copies at the
+// end of the call, each a launch of its own.
 __device__ __forceinline__ void zz_topk_gates(const ZzTopkArgs &a, int s, ZzTopkWaveHdr &h, double cj, float pj,
                                               bool write) {
     const int K = a.K, l = threadIdx.x & 63;
@@ -137,6 +139,8 @@ __device__ __forceinline__ void zz_topk_gates(const ZzTopkArgs &a, int s, ZzTopk
             a.eidx[(size_t)s * K + l] = ej;
             a.ewt[(size_t)s * K + l] = out;
             if (a.topv) a.topv[(size_t)s * K + l] = h.topv[l];
+            if (a.eidx_out) a.eidx_out[(size_t)s * K + l] = ej;
+            if (a.ewt_out) a.ewt_out[(size_t)s * K + l] = out;
         }
     }
     zz_wave_sync_lds();
