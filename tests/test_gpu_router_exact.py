@@ -296,3 +296,15 @@ def test_certified_double_logits(dev, kind, S, cancel):
     bad = got.astype(np.float32).view(np.uint32) != want.dump["logits"].view(np.uint32)
     assert not bad.any(), (int(bad.sum()), np.argwhere(bad)[:4])
     check(L, (out, eidx, ewt), want, exact_weights=True)
+
+
+# ------------------------------------------------- where the batched logits change kernel
+@pytest.mark.parametrize("kind,E,last", [("lfm", 16, 768), ("ling", 128, 96), ("maple", 256, 48)])
+def test_logits_on_both_sides_of_the_rule(dev, kind, E, last):
+    """One wave per logit up to S * E = 12288, the serial chains from there on: ids and
+    gate weights bit-exact on both sides, and from 16 tokens up."""
+    L = Z.make_layer(kind, seed=19, E=E, D=576, MI=64, K=2)
+    for S in (16, 33, last, last + 1):
+        say(f"rule {kind} E={E} S={S}")
+        got, want, ds = run(L, Z.make_input(L, S, 90 + S))
+        check(L, got, want, exact_weights=True)

@@ -33,7 +33,7 @@ static int g_ready = 0;
 // batches of at most this many tokens take the three-launch decode path
 // (ZZ_DECODE_MAX_S, 0 turns it off; never above ZZ_DEC_MAXS)
 static int g_dec_max_s = ZZ_DEC_MAXS;
-static int g_exact_min_s = 16;          // ZZ_EXACT_LOGITS_MIN_S
+static int g_exact_min_s = 0;           // ZZ_EXACT_LOGITS_MIN_S; 0: exact_min_s's rule
 static char g_name[128] = "none";
 static hipStream_t g_stream = nullptr;
 static unsigned *g_diag = nullptr;          // device counters, see zz_moe_stats
@@ -78,7 +78,7 @@ extern "C" int gpu_init(void) {
     ZZ_CHECK(hipMalloc(&g_diag, 16 * sizeof(unsigned)));
     ZZ_CHECK(hipMemset(g_diag, 0, 16 * sizeof(unsigned)));
     // batches from this size on take the exact serial router chains, smaller ones the
-    // certified parallel logits with exact replay of contested chains
+    // certified parallel logits with exact replay of contested chains (0: exact_min_s)
     const char *em = getenv("ZZ_EXACT_LOGITS_MIN_S");
     if (em) g_exact_min_s = atoi(em) < 1 ? 1 : atoi(em);
     const char *dm = getenv("ZZ_DECODE_MAX_S");
@@ -528,6 +528,21 @@ static bool takes_decode(const zz_moe_desc &d, int S) {
     return S <= g_dec_max_s && S <= lim && zz_dec_fits(S, d.K, d.MI);
 }
 
+// The smallest batch whose router logits are the exact serial chains, one lane each,
+// instead of one wave per logit. The chains take their latency (24 us at D = 2048)
+// whatever the batch; the waves' time grows with S * E. The double-chain routers' waves
+// give the same floats: a logit whose rounding they cannot certify is replayed (one in
+// 10^4 to 10^6). Layer us, waves against chains: Ling (E 128) S = 21 70 / 89, 61 90 / 100,
+// 96 94 / 102, 192 113 / 107; LFM (E 32) S = 64 79 / 98, 256 116 / 125, 384 145 / 152, 512
+// 160 / 159; Maple (E 256) S = 32 112 / 131, 48 133 / 146, 61 151 / 159, 96 181 / 179.
+// 12288 waves are Maple's 48, Ling's 96 and LFM's 384. Gemma's waves bound an fp32 chain,
+// far more loosely: from about 16 tokens on most batches would replay one, which takes as
+// long as the chains (S = 16 82 / 90, 21 127 / 90).
+static int exact_min_s(const zz_moe_desc &d) {
+    if (g_exact_min_s) return g_exact_min_s;
+    return d.gating == ZZ_GATE_SOFTMAX_PES ? 16 : 12288 / d.E + 1;
+}
+
 // Kernel arguments of one chunk of S <= chunk_tokens rows of layer L.
 struct ChunkArgs {
     ZzPrepArgs pa;
@@ -561,7 +576,7 @@ static ChunkArgs chunk_args(Layer *L, Workspace &w, const float *d_in, int S, in
     ZzLogitArgs &la = c.la;
     la.D = d.D; la.E = d.E; la.gating = d.gating; la.S = S; la.router = L->router; la.xn = w.xn; la.x = d_in;
     la.bias = c.gemma && d.use_bias ? L->bias : nullptr; la.cen = w.cen; la.bnd = w.bnd; la.diag = g_diag;
-    la.exact_min_s = g_exact_min_s;
+    la.exact_min_s = exact_min_s(d);
 
     ZzTopkArgs &ta = c.ta;
     ta.D = d.D; ta.E = d.E; ta.K = d.K; ta.gating = d.gating; ta.norm_topk = d.norm_topk;

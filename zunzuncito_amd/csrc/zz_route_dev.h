@@ -262,31 +262,39 @@ __device__ void zz_logit_wave_f64(const ZzLogitArgs &a, int s, int e, double *tb
     const float lo = (float)(carry - b), hi = (float)(carry + b);
     float v = lo;
     if (__builtin_amdgcn_readfirstlane(lo != hi)) {
-        // replay, reference order, from the products staged chunk by chunk
-        double r = 0.0, q0 = 0.0, q1 = 0.0, q2 = 0.0, q3 = 0.0, q4 = 0.0, q5 = 0.0, q6 = 0.0, q7 = 0.0;
+        // replay, reference order, from the products staged chunk by chunk, 8 or 16 read
+        // from LDS ahead of their adds. ling's eight accumulators sit in eight lanes (one
+        // lane held all eight: two LDS latencies a step of eight). D % 64 == 0.
+        double r = 0.0;
         for (int c0 = 0; c0 < D; c0 += 64 * ZZ_DPER) {
             zz_stage_products(w, xv, D, c0, tb);
-            if (l == 0) {
-                const int n = min(64 * ZZ_DPER, D - c0);
-                if (grp) {                                 // D % 8 == 0, c0 % 8 == 0
-                    for (int i = 0; i < n; i += 8) {
-                        const double *t = tb + (i / ZZ_DPER) * (ZZ_DPER + 1) + i % ZZ_DPER;
-                        q0 += t[0]; q1 += t[1]; q2 += t[2]; q3 += t[3];
-                        q4 += t[4]; q5 += t[5]; q6 += t[6]; q7 += t[7];
-                    }
-                } else {
-                    for (int i = 0; i < n; i += ZZ_DPER) {
-                        const double *t = tb + (i / ZZ_DPER) * (ZZ_DPER + 1);
-                        const int m = min(ZZ_DPER, n - i);
+            const int n = min(64 * ZZ_DPER, D - c0);
+            if (grp && l < 8) {                            // lane k: accumulator k
+                for (int i = 0; i < n; i += 64) {
+                    double t[8];
 #pragma unroll
-                        for (int k = 0; k < ZZ_DPER; k++)
-                            if (k < m) r += t[k];
+                    for (int k = 0; k < 8; k++) {
+                        const int q = i + 8 * k + l;
+                        t[k] = tb[(q / ZZ_DPER) * (ZZ_DPER + 1) + q % ZZ_DPER];
                     }
+#pragma unroll
+                    for (int k = 0; k < 8; k++) r += t[k];
+                }
+            } else if (!grp && l == 0) {
+                for (int i = 0; i < n; i += ZZ_DPER) {
+                    const double *tp = tb + (i / ZZ_DPER) * (ZZ_DPER + 1);
+                    double t[ZZ_DPER];
+#pragma unroll
+                    for (int k = 0; k < ZZ_DPER; k++) t[k] = tp[k];
+#pragma unroll
+                    for (int k = 0; k < ZZ_DPER; k++) r += t[k];
                 }
             }
             zz_wave_sync_lds();
         }
-        if (grp) r = ((q0 + q1) + (q2 + q3)) + ((q4 + q5) + (q6 + q7));
+        if (grp)
+            r = ((zz_lane_f64(r, 0) + zz_lane_f64(r, 1)) + (zz_lane_f64(r, 2) + zz_lane_f64(r, 3))) +
+                ((zz_lane_f64(r, 4) + zz_lane_f64(r, 5)) + (zz_lane_f64(r, 6) + zz_lane_f64(r, 7)));
         v = (float)r;
         if (l == 0) atomicAdd(a.diag + 1, 1u);
     }
