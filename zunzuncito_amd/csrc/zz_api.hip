@@ -140,6 +140,25 @@ static int grow(float **p, size_t *cap, size_t n) {
     return 1;
 }
 
+// Pinned staging of gpu_matmul, one fixed allocation: calls whose x and y are each up to
+// MM_STAGE floats (1 MiB) have a kernel fetch x from it and the product store y into it.
+// Larger ones, where the bytes and not the two copies' fixed cost count, keep the copies.
+#define MM_STAGE ((size_t)1 << 18)
+static float *g_hx = nullptr, *g_hy = nullptr;
+
+static bool mm_stage() {
+    if (!g_hx) {
+        float *p = nullptr;
+        if (hipHostMalloc((void **)&p, 2 * MM_STAGE * sizeof(float), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();             // the copies serve
+            return false;
+        }
+        g_hx = p;
+        g_hy = p + MM_STAGE;
+    }
+    return true;
+}
+
 extern "C" int gpu_matmul(int fmt, float *y, const uint8_t *W, const float *x, int O, int I, int S) {
     if (!g_ready) ZZ_FAIL("gpu_matmul: not ready");
     if (fmt != ZZ_FMT_Q40 && fmt != ZZ_FMT_Q80 && fmt != ZZ_FMT_TQ2 && fmt != ZZ_FMT_Q4A)
@@ -150,17 +169,31 @@ extern "C" int gpu_matmul(int fmt, float *y, const uint8_t *W, const float *x, i
     ZzRange *m = g_maps.find(W, wb);
     if (!m) ZZ_FAIL("gpu_matmul: W not inside a gpu_map'd range");
     const size_t off = (uintptr_t)W - m->host;
-    if (zz_fp_changed(*m, off, wb)) {            // refilled since its upload: refresh it
+    const uint8_t *dW = m->dev + off;
+    const size_t nx = (size_t)S * I, ny = (size_t)S * O;
+    if (!grow(&g_mx, &g_mxn, nx)) return 0;
+    const bool stage = nx <= MM_STAGE && ny <= MM_STAGE && mm_stage();
+    if (!stage && !grow(&g_my, &g_myn, ny)) return 0;
+    float *out = stage ? g_hy : g_my;
+    if (stage) {
+        memcpy(g_hx, x, sizeof(float) * nx);
+        if (!zz_launch_copy_f32(g_mx, g_hx, nx, g_stream)) ZZ_FAIL("gpu_matmul: launch failed");
+    } else {
+        ZZ_CHECK(hipMemcpyAsync(g_mx, x, sizeof(float) * nx, hipMemcpyHostToDevice, g_stream));
+    }
+    if (!zz_launch_matmul_f32(fmt, out, dW, g_mx, O, I, S, g_stream)) ZZ_FAIL("gpu_matmul: launch failed");
+    // the fingerprint is read while the product runs; a tensor refilled since its upload is
+    // refreshed and the product, not yet handed out, formed again
+    if (zz_fp_changed(*m, off, wb)) {
+        ZZ_CHECK(hipStreamSynchronize(g_stream));
         ZZ_CHECK(hipMemcpy(m->dev + off, W, wb, hipMemcpyHostToDevice));
         zz_fp_take(*m, off, wb);
         g_map_refreshes++;
+        if (!zz_launch_matmul_f32(fmt, out, dW, g_mx, O, I, S, g_stream)) ZZ_FAIL("gpu_matmul: launch failed");
     }
-    const uint8_t *dW = m->dev + off;
-    if (!grow(&g_mx, &g_mxn, (size_t)S * I) || !grow(&g_my, &g_myn, (size_t)S * O)) return 0;
-    ZZ_CHECK(hipMemcpyAsync(g_mx, x, sizeof(float) * (size_t)S * I, hipMemcpyHostToDevice, g_stream));
-    if (!zz_launch_matmul_f32(fmt, g_my, dW, g_mx, O, I, S, g_stream)) ZZ_FAIL("gpu_matmul: launch failed");
     ZZ_CHECK(hipStreamSynchronize(g_stream));
-    ZZ_CHECK(hipMemcpy(y, g_my, sizeof(float) * (size_t)S * O, hipMemcpyDeviceToHost));
+    if (stage) memcpy(y, g_hy, sizeof(float) * ny);
+    else ZZ_CHECK(hipMemcpy(y, g_my, sizeof(float) * ny, hipMemcpyDeviceToHost));
     return 1;
 }
 

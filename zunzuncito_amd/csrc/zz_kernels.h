@@ -234,6 +234,9 @@ int zz_launch_combine(const ZzCombineArgs &a, int S, hipStream_t st);
 int zz_launch_repack(const ZzRepackArgs &a, hipStream_t st);
 // the first n tensors of a.lay only (gate, then up, then down)
 int zz_launch_repack_n(const ZzRepackArgs &a, int n, hipStream_t st);
+// dst[0..n) = src[0..n), n a multiple of 4, both 16-byte aligned
+int zz_launch_copy_f32(float *dst, const float *src, size_t n, hipStream_t st);
+
 // y[S,O] = W[O,I] x[S,I] with f32 activations (gpu.h matmul contract)
 int zz_launch_matmul_f32(int fmt, float *y, const uint8_t *W, const float *x, int O, int I,
                          int S, hipStream_t st);
