@@ -234,7 +234,7 @@ int zz_launch_combine(const ZzCombineArgs &a, int S, hipStream_t st);
 int zz_launch_repack(const ZzRepackArgs &a, hipStream_t st);
 // the first n tensors of a.lay only (gate, then up, then down)
 int zz_launch_repack_n(const ZzRepackArgs &a, int n, hipStream_t st);
-// dst[0..n) = src[0..n), n a multiple of 4, both 16-byte aligned
+// dst[0..n) = src[0..n) in 16-byte pieces: both aligned, and as long as n rounded up to 4
 int zz_launch_copy_f32(float *dst, const float *src, size_t n, hipStream_t st);
 
 // y[S,O] = W[O,I] x[S,I] with f32 activations (gpu.h matmul contract)

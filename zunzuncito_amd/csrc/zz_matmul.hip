@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void zz_copy_f32_kernel(float4 *dst, const flo
 }
 
 int zz_launch_copy_f32(float *dst, const float *src, size_t n, hipStream_t st) {
-    const unsigned n4 = (unsigned)(n / 4);
+    const unsigned n4 = (unsigned)((n + 3) / 4);
     hipLaunchKernelGGL(zz_copy_f32_kernel, dim3((n4 + 255) / 256), dim3(256), 0, st, (float4 *)dst, (const float4 *)src, n4);
     return hipGetLastError() == hipSuccess;
 }
