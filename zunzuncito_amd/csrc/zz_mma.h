@@ -110,10 +110,12 @@ __device__ __forceinline__ float mm_dw(uint2 s, int j, int r) {
 
 // The matrix cores add the block's dot to an integer C operand. With C the bits of the
 // float MM_M = 1.5 * 2^23 the result's bits are the float MM_M + dot, exactly: every dot
-// here is below 2^20 in magnitude (q4_0 16 * 8 * 127 * 32, q8_0 127 * 127 * 32), and from
+// here is below 2^20 in magnitude (q4_0 16 * 8 * 127 * 32, q8_0 128 * 127 * 32), and from
 // 2^23 to 2^24 a float's unit is 1. fma(MM_M + dot, d_w, -MM_M * d_w) then is d_w * dot
-// rounded once: -MM_M * d_w is exact (3 * 2^22 times fp16's 11 bits), so the product needs
-// no integer conversion. tq2 has no block scale and keeps the conversion.
+// rounded once, for every finite d_w: -MM_M * d_w is exact (3 * 2^22 times fp16's 11 bits),
+// so the product needs no integer conversion. An infinite d_w gives inf - inf, a NaN that
+// stays in its sum to the end, where mm_redo forms it again. tq2 has no block scale and
+// keeps the conversion.
 #define MM_MBITS 0x4B400000
 #define MM_M 12582912.0f
 
@@ -245,6 +247,48 @@ __device__ __forceinline__ void mm_store_x(const MmX &x, MmStage &st) {
     for (int k = 0; k < MM_SP; k++) {
         const int i = tid + 256 * k;
         st.s[i >> 2][i & 3] = x.s[k];
+    }
+}
+
+// Sums that ended as a NaN, formed again as d_w * d_x times the plain dot: the signed
+// infinities of an infinite d_w, as the 4x4x4 and decode forms give them. Infinite scales
+// are what the quantisers write where a weight overflows fp16; without one a call pays a
+// compare for every two sums. Each wave for itself, straight from memory and without a
+// barrier, so that its workgroup's other waves need not take part; one tile and block at a
+// time, in fewer registers than the timed loop.
+// row(t), srow(t): the int8 row and block scales of the item's token t.
+template <int FMT, int NT, typename RF, typename SF>
+__device__ __forceinline__ void mm_redo(const uint8_t *E, const ZzTensor &T, int g, RF row, SF srow,
+                                        float (&acc)[NT][4]) {
+    bool nan = false;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+        nan |= __builtin_isunordered(acc[t][0], acc[t][1]) | __builtin_isunordered(acc[t][2], acc[t][3]);
+    if (__builtin_expect(__ballot(nan) == 0ull, 1)) return;
+    const int l = threadIdx.x & 63, qq = l >> 4, nb = T.I / ZZ_BLK;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const ZzWalk W = zz_walk(T, g, l, l & 15);
+        const zz_v4i zero = {0, 0, 0, 0};
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int c = 0; 4 * c < nb; c++) {
+            const MmA A = mm_load_a<FMT>(E, T, W, g, c, l);
+            const bool full = c < W.nfull;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (j >= 2 && !full) continue;
+                const int b = 4 * c + j;
+                const float dw = full ? mm_dw<true>(A.s, j, l) : mm_dw<false>(A.s, j, l);
+                const long x = *(const long *)(row(16 * t + (l & 15)) + b * ZZ_BLK + 8 * qq);
+                const zz_v4i r = __builtin_amdgcn_mfma_i32_16x16x32_i8(x, mm_frag<FMT>(A, j, l), zero, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[i] = fmaf(dw * srow(16 * t + 4 * qq + i)[b], (float)r[i], v[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (acc[t][i] != acc[t][i]) acc[t][i] = v[i];
     }
 }
 

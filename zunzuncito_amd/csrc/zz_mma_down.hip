@@ -53,6 +53,9 @@ __device__ __forceinline__ void mm_down_body(const ZzFfnArgs &a, const ZzItem &i
     // q4_0: the 16*(q - 8) weights; tq2: the row alpha, read now, used at the end
     const float f = FMT == ZZ_FMT_Q40 ? 0.0625f : FMT == ZZ_FMT_TQ2 ? ((const float *)(E + T.off_s))[row] * -0.015625f : 1.0f;
     mm_kloop<FMT, NT, MM_RING, MM_XD(FMT)>(E, T, g, src, sm.st, acc, dbgc);
+    if constexpr (FMT != ZZ_FMT_TQ2)
+        mm_redo<FMT, NT>(E, T, g, [&](int t) { return src.xb + (size_t)(item.p0 + min(t, n - 1)) * MI; },
+                         [&](int t) { return a.hs + (size_t)(item.p0 + min(t, n - 1)) * nb; }, acc);
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll

@@ -57,6 +57,12 @@ __device__ __forceinline__ void mm_up_body(const ZzFfnArgs &a, const ZzItem &ite
     if (GF == ZZ_FMT_TQ2) f = ((const float *)(E + T.off_s))[16 * g + (l & 15)] * -0.015625f;   // used after the K loop
     if (GF == UF || w < 2) mm_kloop<GF, NT, MM_RING, MM_XD(GF)>(E, T, g, src, sm.st, acc, dbgc);
     else mm_kloop<UF, NT, MM_RING, MM_XD(UF)>(E, T, g, src, sm.st, acc, dbgc);
+    if constexpr (GF != ZZ_FMT_TQ2) {
+        auto row = [&](int t) { return src.xb + (size_t)tok[t] * D; };
+        auto srow = [&](int t) { return a.xs + (size_t)tok[t] * nb; };
+        if (GF == UF || w < 2) mm_redo<GF, NT>(E, T, g, row, srow, acc);
+        else mm_redo<UF, NT>(E, T, g, row, srow, acc);
+    }
     if ((w < 2 ? GF : UF) == ZZ_FMT_Q40) f = 0.0625f;     // the 16*(q - 8) weights
     __syncthreads();                             // the stages are done with
 #pragma unroll
