@@ -40,3 +40,17 @@ def test_short_chunks_and_tiles(dev, kind, fmts):
                 check_dots(L, m, x, f"{kind} {fmts} S={S}")
     finally:
         m.close()
+
+
+def test_tq2_large_sums(dev):
+    """Ternary dots of up to 3e38: the sums are of the dots themselves, so what is finite in
+    the reference (whose clamp then makes it an ordinary hidden value) stays finite."""
+    L = Z.make_layer("maple", seed=29, E=4, K=2, D=1088, MI=320)
+    m = gpu_layer(L)
+    try:
+        for S in (3, 6, 20, 50, 130):
+            print("case large sums", S, flush=True)
+            x = Z.make_input(L, S, 31) * np.float32(5e35)
+            check_layer(m, L, x, Z.oracle_moe(L, x))
+    finally:
+        m.close()

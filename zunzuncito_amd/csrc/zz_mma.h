@@ -95,7 +95,7 @@ __device__ __forceinline__ long mm_frag(const MmA &A, int j, int l) {
     // 2*(j&1), k 16..31 plane 2*(j&1)+1, byte k%16 (tq2.h:46-51). mm_chunk flips bit 0 of
     // every code c: c ^ 1 is 1 - c in two bits of two's complement for every c (0..3), and
     // moved to the top of its byte it is the int8 -64 (c - 1), two operations per four
-    // weights (forming c - 1 itself took four).
+    // weights (forming c - 1 itself took four). mm_chunk's product takes the -64 out.
     const uint2 v = j < 2 ? make_uint2(A.q.x, A.q.y) : make_uint2(A.q.z, A.q.w);
     const unsigned sh = 6 - 4 * (j & 1) - 2 * (l >> 5);
     return (long)((unsigned long)((v.x << sh) & 0xC0C0C0C0u) | ((unsigned long)((v.y << sh) & 0xC0C0C0C0u) << 32));
@@ -110,14 +110,21 @@ __device__ __forceinline__ float mm_dw(uint2 s, int j, int r) {
 
 // The matrix cores add the block's dot to an integer C operand. With C the bits of the
 // float MM_M = 1.5 * 2^23 the result's bits are the float MM_M + dot, exactly: every dot
-// here is below 2^20 in magnitude (q4_0 16 * 8 * 127 * 32, q8_0 128 * 127 * 32), and from
+// here is below 2^20 in magnitude (q4_0 16 * 8 * 127 * 32, q8_0 128 * 127 * 32, tq2 128 * 127 * 32), and from
 // 2^23 to 2^24 a float's unit is 1. fma(MM_M + dot, d_w, -MM_M * d_w) then is d_w * dot
 // rounded once, for every finite d_w: -MM_M * d_w is exact (3 * 2^22 times fp16's 11 bits),
 // so the product needs no integer conversion. An infinite d_w gives inf - inf, a NaN that
-// stays in its sum to the end, where mm_redo forms it again. tq2 has no block scale and
-// keeps the conversion.
+// stays in its sum to the end, where mm_redo forms it again. tq2 has no block scale: its
+// d_w is the -1/64 that mm_frag's codes leave, exact like the rest, so that the sums are of
+// the dots themselves (64 times them would overflow where the reference does not).
 #define MM_MBITS 0x4B400000
 #define MM_M 12582912.0f
+
+// the block's dot from a matrix-core result
+template <int FMT>
+__device__ __forceinline__ int mm_dot(int r) {
+    return FMT == ZZ_FMT_TQ2 ? (MM_MBITS - r) / 64 : r - MM_MBITS;
+}
 
 // acc[i] += p[i] * (lane J0 + i's value of sx, in each row of 16 lanes). The compiler
 // leaves the broadcast a move of its own (a third operation per output), so the
@@ -142,15 +149,15 @@ __device__ __forceinline__ void mm_fmac4(float (&acc)[4], const float (&p)[4], f
 // l%16 of its group, VGPR i of tile t token 16t + 4(l/16) + i; lane 16qq + n of sx holds
 // the d_x of token 16(n/4) + 4qq + n%4, so that token's d_x reaches the lanes of its
 // quarter as the DPP row broadcast of lane 4t + i, folded into the multiply-add.
-template <int FMT, int NT, int t = 0>
+template <int NT, int t = 0>
 __device__ __forceinline__ void mm_epi(float (&acc)[NT][4], const zz_v4i (&r)[NT], float dw, float nm, float sx) {
     if constexpr (t < NT) {
         float p[4];
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            p[i] = FMT == ZZ_FMT_TQ2 ? (float)r[t][i] : fmaf(__int_as_float(r[t][i]), dw, nm);
+            p[i] = fmaf(__int_as_float(r[t][i]), dw, nm);
         mm_fmac4<t>(acc[t], p, sx);
-        mm_epi<FMT, NT, t + 1>(acc, r, dw, nm, sx);
+        mm_epi<NT, t + 1>(acc, r, dw, nm, sx);
     }
 }
 
@@ -165,12 +172,11 @@ __device__ __forceinline__ void mm_epi(float (&acc)[NT][4], const zz_v4i (&r)[NT
 // matrix-core instruction against 10.7 over the whole up kernel. Gemma-4 layer, S = 512,
 // Zipf routing: ffn_up 94.8 -> 86.1 us, ffn_down 61.1 -> 58.2; LFM S = 256 61.0 -> 51.5 and
 // 44.2 -> 38.9; Maple (tq2) S = 512 95.7 -> 86.4 and 59.5 -> 55.6 (HIP events).
-// DF(j, r): called with block j's int32 results, MM_MBITS added to each except tq2's
-// (diagnostics builds store them; the timed build passes a hook that does nothing).
+// DF(j, r): called with block j's int32 results as mm_dot takes them (diagnostics builds
+// store them; the timed build passes a hook that does nothing).
 template <int FMT, int NT, bool FULL, typename XF, typename DF>
 __device__ __forceinline__ void mm_chunk(MmA A, int l, float (&acc)[NT][4], XF X, const float4 &sx4, DF dbg) {
-    constexpr int C0 = FMT == ZZ_FMT_TQ2 ? 0 : MM_MBITS;
-    const zz_v4i c0 = {C0, C0, C0, C0};
+    const zz_v4i c0 = {MM_MBITS, MM_MBITS, MM_MBITS, MM_MBITS};
     const float sx[4] = {sx4.x, sx4.y, sx4.z, sx4.w};
     if (FMT == ZZ_FMT_TQ2)                       // here, not at the load: that would wait for it
         A.q = make_uint4(A.q.x ^ 0x55555555u, A.q.y ^ 0x55555555u, A.q.z ^ 0x55555555u, A.q.w ^ 0x55555555u);
@@ -186,7 +192,7 @@ __device__ __forceinline__ void mm_chunk(MmA A, int l, float (&acc)[NT][4], XF X
 #pragma unroll
         for (int t = 0; t < NT; t++) r[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(B[t], fw, c0, 0, 0, 0);
         dbg(j, r);
-        float dw = 1.0f, nm = 0.0f;
+        float dw = -0.015625f, nm = 0.015625f * MM_M;
         if constexpr (FMT != ZZ_FMT_TQ2) {
             // the empty asm keeps the conversion from being folded into each product as
             // the slower mixed-precision v_fma_mix_f32
@@ -194,7 +200,7 @@ __device__ __forceinline__ void mm_chunk(MmA A, int l, float (&acc)[NT][4], XF X
             asm("" : "+v"(dw));
             nm = dw * -MM_M;
         }
-        mm_epi<FMT, NT>(acc, r, dw, nm, sx[j]);
+        mm_epi<NT>(acc, r, dw, nm, sx[j]);
         // three or four tiles (q8_0 two): one block at a time (the next block's LDS reads
         // hoisted over this one would hold NT more operand registers: q8_0 spilled 28);
         // fewer leave the scheduler free to overlap them (0.5 us off each FFN kernel at
@@ -355,8 +361,12 @@ __device__ __forceinline__ void mm_kloop(const uint8_t *E, const ZzTensor &T, in
 
 // Weight ring and activation depth. With one weight row a lane its chunk takes 6 (q4_0) or
 // 10 (q8_0) registers instead of 12 and 16, which pays for four sets at every tile count
-// (three before, from three tiles on) and, but for q8_0, for activations two chunks ahead:
-// Maple S = 512 ffn_up 90.1 us with three sets and one chunk ahead, 85.7 with these.
+// (three before, from three tiles on) and, but for q8_0, for activations two chunks ahead.
+// tq2 always took 4 registers a chunk, so its four-tile bodies hold a few values too many
+// (the compiler keeps 14 in scratch in down, 7 in up, outside the K loop), and it is the
+// fastest of the depths all the same: Maple S = 512 up 84.4 / down 54.3 us, with activations
+// one chunk ahead and nothing in scratch 85.9 / 56.0, with three sets as well 85.4 / 56.3;
+// S = 128 74.3 / 50.2, 75.4 / 50.3, 75.7 / 49.8 (HIP events).
 #define MM_RING 4
 #define MM_XD(FMT) ((FMT) == ZZ_FMT_Q80 ? 1 : 2)
 

@@ -43,15 +43,14 @@ __device__ __forceinline__ void mm_down_body(const ZzFfnArgs &a, const ZzItem &i
                 for (int i = 0; i < 4; i++) {
                     const int tk = 16 * t + 4 * qq + i;
                     if (tk < n)
-                        mm_dbg_dn(a, item.p0 + tk, 16 * g + (l & 15), 4 * c + j,
-                                  FMT == ZZ_FMT_TQ2 ? -rr[t][i] / 64 : rr[t][i] - MM_MBITS);
+                        mm_dbg_dn(a, item.p0 + tk, 16 * g + (l & 15), 4 * c + j, mm_dot<FMT>(rr[t][i]));
                 }
         }
     };
     float acc[NT][4];
     const int row = 16 * g + (l & 15);
     // q4_0: the 16*(q - 8) weights; tq2: the row alpha, read now, used at the end
-    const float f = FMT == ZZ_FMT_Q40 ? 0.0625f : FMT == ZZ_FMT_TQ2 ? ((const float *)(E + T.off_s))[row] * -0.015625f : 1.0f;
+    const float f = FMT == ZZ_FMT_Q40 ? 0.0625f : FMT == ZZ_FMT_TQ2 ? ((const float *)(E + T.off_s))[row] : 1.0f;
     mm_kloop<FMT, NT, MM_RING, MM_XD(FMT)>(E, T, g, src, sm.st, acc, dbgc);
     if constexpr (FMT != ZZ_FMT_TQ2)
         mm_redo<FMT, NT>(E, T, g, [&](int t) { return src.xb + (size_t)(item.p0 + min(t, n - 1)) * MI; },

@@ -48,13 +48,13 @@ __device__ __forceinline__ void mm_up_body(const ZzFfnArgs &a, const ZzItem &ite
                     const int tk = 16 * t + 4 * qq + i;
                     if (tk < n)
                         mm_dbg_up(a, item.p0 + tk, w < 2 ? 0 : 1, 16 * g + (l & 15), 4 * c + j,
-                                  GF == ZZ_FMT_TQ2 ? -rr[t][i] / 64 : rr[t][i] - MM_MBITS);
+                                  mm_dot<GF>(rr[t][i]));
                 }
         }
     };
     float acc[NT][4];
     float f = 1.0f;                              // tq2.h:154, alpha of the row: read now,
-    if (GF == ZZ_FMT_TQ2) f = ((const float *)(E + T.off_s))[16 * g + (l & 15)] * -0.015625f;   // used after the K loop
+    if (GF == ZZ_FMT_TQ2) f = ((const float *)(E + T.off_s))[16 * g + (l & 15)];   // used after the K loop
     if (GF == UF || w < 2) mm_kloop<GF, NT, MM_RING, MM_XD(GF)>(E, T, g, src, sm.st, acc, dbgc);
     else mm_kloop<UF, NT, MM_RING, MM_XD(UF)>(E, T, g, src, sm.st, acc, dbgc);
     if constexpr (GF != ZZ_FMT_TQ2) {
