@@ -115,7 +115,10 @@ __global__ __launch_bounds__(256) void zz_dec_logits_kernel(ZzDecRouteArgs a) {
     const ZzPrepArgs &pp = a.prep;
     const ZzLogitArgs &lg = a.lg;
     const int S = a.S, D = pp.D, nb = D / ZZ_BLK, tid = threadIdx.x, e = blockIdx.x;
-    const bool gem = pp.gemma;
+    // only gemma's blocks defer their combine: those forms hold no code of the f64 routers.
+    // With it this kernel took 11.4 us of a stack's block, without it 10.3 (kernel trace; the
+    // registers are the same), and four blocks under the full head 251.4 us against 245.9.
+    const bool gem = FIN || pp.gemma;
     // gemma: the D rounded products (padded); lfm/maple/ling: one product buffer per
     // token's wave
     __shared__ __attribute__((aligned(16))) char sbuf[(ZZ_MAXD + ZZ_MAXD / 32) * 4 > DEC_MAXS * ZZ_DBUF * 8
@@ -193,7 +196,6 @@ __global__ __launch_bounds__(256) void zz_dec_logits_kernel(ZzDecRouteArgs a) {
                                 lg.bnd + (size_t)s * lg.E + e);
         }
     } else {
-        if (FIN) combine();
         if ((tid >> 6) < S) zz_logit_wave_f64(lg, tid >> 6, e, (double *)sbuf + (tid >> 6) * ZZ_DBUF);
     }
     // the expert input quantisation: block g on workgroup g % E, lanes 8(g / E)..+7;
@@ -758,6 +760,7 @@ __global__ __launch_bounds__(256) void zz_dec_norm_kernel(float *out, const floa
 int zz_launch_dec_logits(const ZzDecRouteArgs &a, hipStream_t st) {
     const int R = (a.prep.D + 255) / 256;
     const dim3 g(a.dense ? 16 : a.lg.E);
+    if (a.fin && !a.prep.gemma) return 0;
     if (a.fin) {                                     // zz_dec_fin_fits holds
         if (R <= 12) hipLaunchKernelGGL((zz_dec_logits_kernel<12, true>), g, dim3(256), 0, st, a);
         else hipLaunchKernelGGL((zz_dec_logits_kernel<16, true>), g, dim3(256), 0, st, a);
