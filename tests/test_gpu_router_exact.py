@@ -308,3 +308,22 @@ def test_logits_on_both_sides_of_the_rule(dev, kind, E, last):
         say(f"rule {kind} E={E} S={S}")
         got, want, ds = run(L, Z.make_input(L, S, 90 + S))
         check(L, got, want, exact_weights=True)
+
+
+@pytest.mark.parametrize("kind", ["lfm", "maple", "ling"])
+@pytest.mark.parametrize("S", [1, 5, 20])
+def test_zero_logits_keep_their_sign(dev, kind, S):
+    """A router row of zeros (and one of negative zeros) sums to +0 in the reference."""
+    say(f"zero rows {kind} S={S}")
+    L = small_layer(kind, seed=23)
+    L.router[3] = 0.0
+    L.router[6] = -0.0
+    x = Z.make_input(L, S, 50 + S)
+    m = gpu_layer(L)
+    try:
+        m.forward(x)
+        got = m.debug(S, logits=True)["logits"]
+    finally:
+        m.close()
+    want = Z.oracle_moe(L, x, dump=True).dump["logits"]
+    assert np.array_equal(got.astype(np.float32).view(np.uint32), want.view(np.uint32))

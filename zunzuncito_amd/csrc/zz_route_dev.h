@@ -260,7 +260,7 @@ __device__ void zz_logit_wave_f64(const ZzLogitArgs &a, int s, int e, double *tb
     }
     b = b * 1.000001 + 1e-300;
     const float lo = (float)(carry - b), hi = (float)(carry + b);
-    float v = lo;
+    float v = (float)carry;                  // lo == hi: theirs, but +0 where b alone made lo -0
     if (__builtin_amdgcn_readfirstlane(lo != hi)) {
         // replay, reference order, from the products staged chunk by chunk, 8 or 16 read
         // from LDS ahead of their adds. ling's eight accumulators sit in eight lanes (one
