@@ -327,3 +327,27 @@ def test_zero_logits_keep_their_sign(dev, kind, S):
         m.close()
     want = Z.oracle_moe(L, x, dump=True).dump["logits"]
     assert np.array_equal(got.astype(np.float32).view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["lfm", "maple", "ling"])
+@pytest.mark.parametrize("S", [3, 21, 200])
+def test_bf16_values_need_no_replay(dev, kind, S):
+    """Inputs and router rows of bf16 values put many logits on a float rounding tie, but
+    their sums are exact in any order: the reference's floats without a serial replay."""
+    say(f"bf16 values {kind} S={S}")
+    L = small_layer(kind, seed=27)
+    bf = lambda v: (np.ascontiguousarray(v, np.float32).view(np.uint32) & 0xffff0000).view(np.float32)
+    L.router = bf(L.router)
+    x = bf(Z.make_input(L, S, 60 + S))
+    m = gpu_layer(L)
+    try:
+        s0 = np.array(zz.stats(), np.int64)
+        out, eidx, ewt = m.forward(x)
+        ds = np.array(zz.stats(), np.int64) - s0
+        got = m.debug(S, logits=True)["logits"]
+    finally:
+        m.close()
+    want = Z.oracle_moe(L, x, dump=True)
+    assert np.array_equal(got.astype(np.float32).view(np.uint32), want.dump["logits"].view(np.uint32))
+    check(L, (out, eidx, ewt), want, exact_weights=True)
+    assert ds[1] == 0, ds.tolist()

@@ -188,7 +188,7 @@ __device__ void zz_tight_block_scan(const float *buf, int D, bool hb, float bz, 
 // contiguous run of the order, and joins the runs by a wave scan: that gives the
 // prefix sums S_i (to gamma_40 T, T = sum |p_i|) and the centre S_D (to gamma_30 T).
 // When every value the bound allows rounds to one float, that float is the
-// reference's logit; otherwise one lane replays the chain from the products staged
+// reference's logit, and so it is when no sum can have been rounded; otherwise one lane replays the chain from the products staged
 // in LDS, chunk by chunk.
 #define ZZ_DPER 16                           // products per lane per chunk
 #define ZZ_DBUF (64 * (ZZ_DPER + 1))         // doubles of one wave's product buffer
@@ -212,6 +212,29 @@ __device__ __forceinline__ void zz_stage_products(const float *w, const float *x
             c0 + q < D ? (double)wv[j] * (double)xr[j] : 0.0;
     }
     zz_wave_sync_lds();
+}
+
+// The exponent of a nonzero finite double's lowest set bit: it is a whole multiple of
+// 2^that. (A product of two floats is never a subnormal double.)
+__device__ __forceinline__ int zz_lowbit_exp(double p) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, p);
+    const unsigned long long m = (u & ((1ull << 52) - 1)) | (1ull << 52);
+    return (int)((u >> 52) & 0x7ff) - 1075 + (__ffsll((long long)m) - 1);
+}
+
+// Whether every partial sum of the products, in any order, is exact in double: all are
+// multiples of 2^q, q their lowest set bit, and T = sum |p_i|, which bounds the partial
+// sums, is below 2^(q + 53). (T itself is then exact; rounded, it would not have fallen
+// below that power of two.) All lanes get the answer.
+__device__ __forceinline__ bool zz_exact_sums(const float *w, const float *x, int D, double T) {
+    const int l = threadIdx.x & 63;
+    int q = 1024;
+    for (int i = l; i < D; i += 64) {                        // D % 64 == 0
+        const double p = (double)w[i] * (double)x[i];
+        if (p != 0.0) q = min(q, zz_lowbit_exp(p));
+    }
+    q = zz_group_reduce<64>(q, [](int a, int b) { return min(a, b); });
+    return T < ldexp(1.0, min(q + 53, 1023));                // false for a NaN or an infinite T
 }
 
 // logit of token s, expert e (router input x), by one wave; tb: ZZ_DBUF doubles of
@@ -261,7 +284,11 @@ __device__ void zz_logit_wave_f64(const ZzLogitArgs &a, int s, int e, double *tb
     b = b * 1.000001 + 1e-300;
     const float lo = (float)(carry - b), hi = (float)(carry + b);
     float v = (float)carry;                  // lo == hi: theirs, but +0 where b alone made lo -0
-    if (__builtin_amdgcn_readfirstlane(lo != hi)) {
+    // A sum on a rounding tie is contested whatever its bound. With f32 inputs and rows one
+    // in 10^4 to 10^6 is; where both hold bf16 values (16-bit products) one in some 200 is,
+    // every batch replayed one, and a LFM layer of S = 256 took 130.7 us where the chains
+    // take 126.6. There all the sums are exact and the centre is the chain's: 121.6 us.
+    if (__builtin_amdgcn_readfirstlane(lo != hi) && !zz_exact_sums(w, xv, D, T)) {
         // replay, reference order, from the products staged chunk by chunk, 8 or 16 read
         // from LDS ahead of their adds. ling's eight accumulators sit in eight lanes (one
         // lane held all eight: two LDS latencies a step of eight). D % 64 == 0.
