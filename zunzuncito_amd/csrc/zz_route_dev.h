@@ -225,16 +225,32 @@ __device__ __forceinline__ int zz_lowbit_exp(double p) {
 // Whether every partial sum of the products, in any order, is exact in double: all are
 // multiples of 2^q, q their lowest set bit, and T = sum |p_i|, which bounds the partial
 // sums, is below 2^(q + 53). (T itself is then exact; rounded, it would not have fallen
-// below that power of two.) All lanes get the answer.
-__device__ __forceinline__ bool zz_exact_sums(const float *w, const float *x, int D, double T) {
+// below that power of two.) All lanes get the answer. tb holds the last chunk's products:
+// f32 values fail at the first of each lane, without another load (walking the row for them
+// took a Ling layer of 21 tokens from 72 to 76 us).
+__device__ __forceinline__ bool zz_exact_sums(const float *w, const float *x, int D, double T, const double *tb) {
     const int l = threadIdx.x & 63;
     int q = 1024;
-    for (int i = l; i < D; i += 64) {                        // D % 64 == 0
-        const double p = (double)w[i] * (double)x[i];
-        if (p != 0.0) q = min(q, zz_lowbit_exp(p));
+    auto low = [&](double p) { q = p != 0.0 ? min(q, zz_lowbit_exp(p)) : q; };
+    auto below = [&] {                                       // false for a NaN or an infinite T
+        q = zz_group_reduce<64>(q, [](int a, int b) { return min(a, b); });
+        return __builtin_amdgcn_readfirstlane(T < ldexp(1.0, min(q + 53, 1023)));
+    };
+    low(tb[l * (ZZ_DPER + 1)]);
+    if (!below()) return false;
+#pragma unroll
+    for (int k = 1; k < ZZ_DPER; k++) low(tb[l * (ZZ_DPER + 1) + k]);
+    for (int c0 = 0; c0 + 64 * ZZ_DPER < D; c0 += 64 * ZZ_DPER) {     // the chunks before it, all full
+        float wv[ZZ_DPER], xr[ZZ_DPER];
+#pragma unroll
+        for (int j = 0; j < ZZ_DPER; j++) {
+            wv[j] = w[c0 + 64 * j + l];
+            xr[j] = x[c0 + 64 * j + l];
+        }
+#pragma unroll
+        for (int j = 0; j < ZZ_DPER; j++) low((double)wv[j] * (double)xr[j]);
     }
-    q = zz_group_reduce<64>(q, [](int a, int b) { return min(a, b); });
-    return T < ldexp(1.0, min(q + 53, 1023));                // false for a NaN or an infinite T
+    return below();
 }
 
 // logit of token s, expert e (router input x), by one wave; tb: ZZ_DBUF doubles of
@@ -288,7 +304,7 @@ __device__ void zz_logit_wave_f64(const ZzLogitArgs &a, int s, int e, double *tb
     // in 10^4 to 10^6 is; where both hold bf16 values (16-bit products) one in some 200 is,
     // every batch replayed one, and a LFM layer of S = 256 took 130.7 us where the chains
     // take 126.6. There all the sums are exact and the centre is the chain's: 121.6 us.
-    if (__builtin_amdgcn_readfirstlane(lo != hi) && !zz_exact_sums(w, xv, D, T)) {
+    if (__builtin_amdgcn_readfirstlane(lo != hi) && !zz_exact_sums(w, xv, D, T, tb)) {
         // replay, reference order, from the products staged chunk by chunk, 8 or 16 read
         // from LDS ahead of their adds. ling's eight accumulators sit in eight lanes (one
         // lane held all eight: two LDS latencies a step of eight). D % 64 == 0.
