@@ -387,12 +387,15 @@ static void zz_launch_logits_exact(const ZzLogitArgs &b, int S, hipStream_t st) 
     else zz_launch_logits_exact_tt<KC, 4>(b, S, st);
 }
 
-// Top-k gating, one wave per token (zz_topk_wave.h), four tokens per workgroup.
+// Top-k gating, one wave per token (zz_topk_wave.h), four tokens per workgroup. A kernel per
+// lane count: as branches of one kernel the four forms spanned 90 KB of code, and a Ling
+// batch of 21 tokens took 9.6 or 10.4 us with where the linker put them.
+template <int EPL>
 __global__ __launch_bounds__(256) void zz_topk_kernel(ZzTopkArgs a, int S) {
     extern __shared__ __attribute__((aligned(16))) char tk_lds[];
     const int w = threadIdx.x >> 6, s = blockIdx.x * 4 + w;
     if (s >= S) return;
-    zz_topk_wave_any(a, s, tk_lds + w * zz_topk_wave_bytes(a.E));
+    zz_topk_wave<EPL>(a, s, tk_lds + w * zz_topk_wave_bytes(a.E), true, true);
 }
 
 // -------------------------------------------------------------------------------
@@ -698,7 +701,14 @@ int zz_launch_logits(const ZzLogitArgs &a, int S, hipStream_t st) {
 }
 
 int zz_launch_topk(const ZzTopkArgs &a, int S, hipStream_t st) {
-    hipLaunchKernelGGL(zz_topk_kernel, dim3((S + 3) / 4), dim3(256), 4 * zz_topk_wave_bytes(a.E), st, a, S);
+    const dim3 g((S + 3) / 4), t(256);
+    const size_t lds = 4 * zz_topk_wave_bytes(a.E);
+    switch (zz_topk_epl(a.E)) {
+    case 1: hipLaunchKernelGGL(zz_topk_kernel<1>, g, t, lds, st, a, S); break;
+    case 2: hipLaunchKernelGGL(zz_topk_kernel<2>, g, t, lds, st, a, S); break;
+    case 4: hipLaunchKernelGGL(zz_topk_kernel<4>, g, t, lds, st, a, S); break;
+    default: hipLaunchKernelGGL(zz_topk_kernel<8>, g, t, lds, st, a, S); break;
+    }
     return hipGetLastError() == hipSuccess;
 }
 
