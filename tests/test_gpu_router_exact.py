@@ -299,15 +299,34 @@ def test_certified_double_logits(dev, kind, S, cancel):
 
 
 # ------------------------------------------------- where the batched logits change kernel
-@pytest.mark.parametrize("kind,E,last", [("lfm", 16, 768), ("ling", 128, 96), ("maple", 256, 48)])
-def test_logits_on_both_sides_of_the_rule(dev, kind, E, last):
-    """One wave per logit up to S * E = 12288, the serial chains from there on: ids and
-    gate weights bit-exact on both sides, and from 16 tokens up."""
-    L = Z.make_layer(kind, seed=19, E=E, D=576, MI=64, K=2)
-    for S in (16, 33, last, last + 1):
-        say(f"rule {kind} E={E} S={S}")
-        got, want, ds = run(L, Z.make_input(L, S, 90 + S))
+@pytest.mark.parametrize("kind,E,D,last", [
+    ("lfm", 32, 512, 128), ("lfm", 32, 1088, 136), ("lfm", 16, 2048, 512), ("maple", 128, 768, 48),
+    ("maple", 256, 512, 24), ("maple", 256, 2048, 48), ("maple", 256, 4096, 48), ("ling", 128, 576, 54),
+    ("ling", 128, 1088, 51), ("ling", 128, 2048, 96), ("lfm", 256, 512, 24), ("ling", 512, 512, 15)])
+def test_logits_on_both_sides_of_the_rule(dev, kind, E, D, last):
+    """One wave per logit up to `last` tokens, the serial chains from there on (a planted
+    rounding tie is replayed by the waves only): logits, ids and gate weights bit-exact on
+    both sides, the tie's too."""
+    L = Z.make_layer(kind, seed=19, E=E, D=D, MI=64, K=2)
+    L.router[5] = 0.0
+    L.router[5, :3] = [1.0, 2.0 ** -24, 2.0 ** -60]
+    for S in (last, last + 1):
+        say(f"rule {kind} E={E} D={D} S={S}")
+        x = Z.make_input(L, S, 90 + S)
+        x[:, :3] = 1.0
+        m = gpu_layer(L)
+        try:
+            s0 = np.array(zz.stats(), np.int64)
+            got = m.forward(x)
+            ds = np.array(zz.stats(), np.int64) - s0
+            logits = m.debug(S, logits=True)["logits"]
+        finally:
+            m.close()
+        want = Z.oracle_moe(L, x, dump=True)
+        bad = logits.astype(np.float32).view(np.uint32) != want.dump["logits"].view(np.uint32)
+        assert not bad.any(), (int(bad.sum()), np.argwhere(bad)[:4])
         check(L, got, want, exact_weights=True)
+        assert ds[1] >= S if S == last else ds[1] == 0, ds.tolist()
 
 
 @pytest.mark.parametrize("kind", ["lfm", "maple", "ling"])

@@ -568,18 +568,27 @@ static bool takes_decode(const zz_moe_desc &d, int S) {
 }
 
 // The smallest batch whose router logits are the exact serial chains, one lane each,
-// instead of one wave per logit. The chains take their latency (24 us at D = 2048)
-// whatever the batch; the waves' time grows with S * E. The double-chain routers' waves
-// give the same floats: a logit whose rounding they cannot certify is replayed (one in
-// 10^4 to 10^6). Layer us, waves against chains: Ling (E 128) S = 21 70 / 89, 61 90 / 100,
-// 96 94 / 102, 192 113 / 107; LFM (E 32) S = 64 79 / 98, 256 116 / 125, 384 145 / 152, 512
-// 160 / 159; Maple (E 256) S = 32 112 / 131, 48 133 / 146, 61 151 / 159, 96 181 / 179.
-// 12288 waves are Maple's 48, Ling's 96 and LFM's 384. Gemma's waves bound an fp32 chain,
-// far more loosely: from about 16 tokens on most batches would replay one, which takes as
-// long as the chains (S = 16 82 / 90, 21 127 / 90).
+// instead of one wave per logit. The chains take their latency (5 us + 10 ns * D, half as
+// much again where E >= 256 has eight tokens share a workgroup) whatever the batch; the
+// waves' time grows with S * E and with the 1024-wide chunks that they walk, full or not.
+// The double-chain routers' waves give the same floats: a logit whose rounding they cannot
+// certify is replayed (one in 10^4 to 10^6). Kernel us, waves against chains, 8192 (12288)
+// logits of one-chain routers: E 32, D 512 14.1 / 10.2 (4096: 9.8), 768 14.8 / 12.7 (6144:
+// 12.8), 1024 15.1 / 15.3 (18.9 / 15.5), 1088 20.7 / 18.2 (4096: 13.7), 2048 25.4 / 26.0
+// (28.5 / 26.2), 4096 40.2 / 45.6 (59.7 / 45.8); E 256, D 512 14.1 / 12.9 (6144: 12.3),
+// 1024 14.9 / 20.4 (18.6 / 20.5), 2048 22.1 / 34.8 (29.3 / 35.4), 4096 38.7 / 63.7 (55.5 /
+// 64.0). The grouped router's waves need no prefix sums: E 128, D 512 12.2 / 10.4 (6144:
+// 10.7), 1024 12.9 / 15.4 (15.9 / 15.5), 2048 20.8 / 26.7 (24.7 / 26.3), 4096 38.7 / 45.7
+// (44.8 / 45.7). Over 512 <= D <= 4096, f32 and bf16 values, the line below loses 0.7 us at
+// most. Gemma's waves bound an fp32 chain, far more loosely: from about 16 tokens on most
+// batches would replay one, which takes as long as the chains (layer us, S = 16 82 / 90, 21
+// 127 / 90).
 static int exact_min_s(const zz_moe_desc &d) {
     if (g_exact_min_s) return g_exact_min_s;
-    return d.gating == ZZ_GATE_SOFTMAX_PES ? 16 : 12288 / d.E + 1;
+    if (d.gating == ZZ_GATE_SOFTMAX_PES) return 16;
+    const int per = d.gating == ZZ_GATE_GROUPED || d.E >= 256 ? 12 : 8;
+    const int s = per * d.D / ((d.D + 1023) / 1024) / d.E + 1;
+    return s < 16 ? 16 : s;
 }
 
 // Kernel arguments of one chunk of S <= chunk_tokens rows of layer L.
