@@ -10,9 +10,11 @@
 // of 8 weights (4 lanes a 32-weight block), so a wave's loads of weights and of x are
 // contiguous and each x value loaded serves MV_R rows, each weight T tokens; the
 // partial sums meet by a transposing wave reduction and LDS. Bound by latency at an
-// engine's sizes: q4_0 2112 x 2816, 5 tokens, 23.2 us -> 16.7 (kernel trace, other work
-// between the calls) against one wave per (row, token) whose lanes read whole blocks byte
-// by byte and every token's wave the weights again.
+// engine's sizes. Against one wave per (row, token) whose lanes read whole blocks byte by
+// byte and every token's wave the weights again, q4_0, kernel trace with other work between
+// the calls: 2112 x 2816, 1 token 8.0 -> 4.9 us, 5 tokens 22.6 -> 7.2, 4096 x 2816, 16
+// tokens 111.5 -> 18.0 (q8_0 9.7 -> 5.4, 25.8 -> 8.1, 127 -> 20.8). It rests on the sums
+// staying in registers: in scratch they made 17.9, 17.9 and 49.9 us.
 #include "zz_common.h"
 #include "zz_kernels.h"
 
@@ -101,9 +103,11 @@ __device__ __forceinline__ void mv_reduce(float (&acc)[N], int l) {
         const bool up = (l >> K) & 1;
 #pragma unroll
         for (int v = 0; v < h; v++) {
-            const float keep = up ? acc[v + h] : acc[v];
+            // both read first: a choice between two elements is a choice of addresses to
+            // the compiler, and the array then lives in scratch or LDS
+            const float lo = acc[v], hi = acc[v + h], keep = up ? hi : lo;
             if constexpr (QUAD && K < 2) acc[v] = keep;
-            else acc[v] = keep + __shfl_xor(up ? acc[v] : acc[v + h], 1 << K);
+            else acc[v] = keep + __shfl_xor(up ? lo : hi, 1 << K);
         }
         mv_reduce<QUAD, h, N, K + 1>(acc, l);
     } else if constexpr ((1 << K) < 64) {
