@@ -2,6 +2,10 @@
 weights, row counts off the workgroup's four, every number of tokens a workgroup takes and
 the calls split over several, tensors that start at an odd byte of their mapping, and
 infinite block scales."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -58,3 +62,38 @@ def test_infinite_scales(dev, fmt, bb):
     ref = np.zeros((S, O), np.float32)
     Z.oracle().orc_matmul_f32(fmt, Z.ptr(ref), Z.ptr(W), Z.ptr(x), O, I, S)
     assert not np.isfinite(ref).any() and np.array_equal(y, ref, equal_nan=True)
+
+
+_CHILD = """
+import numpy as np
+import zunzuncito_amd as zz
+
+def maps():
+    return {l.split()[0] for l in open("/proc/self/maps") if "/dev/dri/" in l}
+
+def product():
+    W = zz.gpu_map(np.full(64 * 2 * 18, 0x44, np.uint8))
+    return zz.gpu_matmul(zz.GPU_FMT_Q40, W, np.ones((3, 64), np.float32), 64, 64)
+
+size = lambda m: int(m.split("-")[1], 16) - int(m.split("-")[0], 16)
+zz.init()
+before = maps()
+y = product()
+staging = {m for m in maps() - before if size(m) == 2 << 20}
+zz.lib().gpu_shutdown()
+print("staging", len(staging), "left", len(staging & maps()), flush=True)
+for _ in range(2):
+    zz.init()
+    assert np.array_equal(product(), y)
+    zz.lib().gpu_shutdown()
+print("done")
+"""
+
+
+def test_shutdown_gives_the_staging_back():
+    """The 2 MiB pinned staging leaves the process with gpu_shutdown, and calls after another
+    gpu_init have theirs again. In a process of its own: a shutdown takes every layer."""
+    r = subprocess.run([sys.executable, "-c", _CHILD], cwd=Z.ROOT, capture_output=True, text=True, timeout=100,
+                       env=dict(os.environ, PYTHONPATH=Z.ROOT))
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
+    assert "staging 1 left 0" in r.stdout, r.stdout

@@ -1044,7 +1044,8 @@ extern "C" void gpu_shutdown(void) {
     g_maps.clear([](const ZzRange &m) { (void)hipFree(m.dev); });
     if (g_mx) (void)hipFree(g_mx);
     if (g_my) (void)hipFree(g_my);
-    g_mx = g_my = nullptr;
+    if (g_hx) (void)hipHostFree(g_hx);           // g_hy is its second half
+    g_mx = g_my = g_hx = g_hy = nullptr;
     g_mxn = g_myn = 0;
     (void)hipFree(g_diag);
     g_diag = nullptr;
