@@ -33,7 +33,7 @@ static int g_ready = 0;
 // batches of at most this many tokens take the three-launch decode path
 // (ZZ_DECODE_MAX_S, 0 turns it off; never above ZZ_DEC_MAXS)
 static int g_dec_max_s = ZZ_DEC_MAXS;
-static int g_exact_min_s = 0;           // ZZ_EXACT_LOGITS_MIN_S; 0: exact_min_s's rule
+static int g_exact_min_s = 0;           // ZZ_EXACT_LOGITS_MIN_S; 0 (unset): exact_min_s's rule
 static char g_name[128] = "none";
 static hipStream_t g_stream = nullptr;
 static unsigned *g_diag = nullptr;          // device counters, see zz_moe_stats
@@ -78,7 +78,8 @@ extern "C" int gpu_init(void) {
     ZZ_CHECK(hipMalloc(&g_diag, 16 * sizeof(unsigned)));
     ZZ_CHECK(hipMemset(g_diag, 0, 16 * sizeof(unsigned)));
     // batches from this size on take the exact serial router chains, smaller ones the
-    // certified parallel logits with exact replay of contested chains (0: exact_min_s)
+    // certified parallel logits with exact replay of contested chains; unset, exact_min_s
+    // draws the line, and values below 1 mean 1
     const char *em = getenv("ZZ_EXACT_LOGITS_MIN_S");
     if (em) g_exact_min_s = atoi(em) < 1 ? 1 : atoi(em);
     const char *dm = getenv("ZZ_DECODE_MAX_S");

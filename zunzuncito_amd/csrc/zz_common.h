@@ -258,9 +258,6 @@ template <typename T>
 __device__ __forceinline__ T zz_rows_sum(T v) {
     return zz_rows_reduce(v, [](T x, T y) { return x + y; });
 }
-__device__ __forceinline__ float zz_rows_max(float v) {
-    return zz_rows_reduce(v, [](float x, float y) { return fmaxf(x, y); });
-}
 
 // inclusive prefix sum over a wave: DPP shifts within each 16-lane row by 1, 2, 4,
 // 8 (lanes shifted in from outside the row add zero), then row_bcast:15 adds row 0's
