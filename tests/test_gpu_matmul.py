@@ -64,6 +64,27 @@ def test_infinite_scales(dev, fmt, bb):
     assert not np.isfinite(ref).any() and np.array_equal(y, ref, equal_nan=True)
 
 
+@pytest.mark.parametrize("fmt", [Z.FMT_Q40, Z.FMT_TQ2])
+@pytest.mark.parametrize("O,I,S", [(64, 4096, 64), (40, 4096, 65), (8191, 64, 33), (4099, 2112, 70)])
+def test_staged_and_copied_calls(dev, fmt, O, I, S):
+    """Up to 2^18 values of x and of y go through the pinned staging (the first shape just
+    does), larger ones by copies (x, y, both); in each the weights are rewritten on the host
+    and the next call forms the product again. Within 1e-5 of the largest output, as above."""
+    print("case", fmt, O, I, S, flush=True)
+    rng = np.random.default_rng(77)
+    Wm = zz.gpu_map(np.array(_weights(rng, fmt, O, I)))
+    for k in range(3):
+        x = rng.standard_normal((S, I)).astype(np.float32)
+        n0 = zz.lib().zz_gpu_map_refreshes()
+        if k == 1:
+            Wm[:] = _weights(rng, fmt, O, I)
+        y = zz.gpu_matmul(fmt, Wm, x, O, I)
+        assert zz.lib().zz_gpu_map_refreshes() - n0 == (k == 1)
+        ref = np.zeros((S, O), np.float32)
+        Z.oracle().orc_matmul_f32(fmt, Z.ptr(ref), Z.ptr(Wm), Z.ptr(x), O, I, S)
+        assert np.abs(y - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
 _CHILD = """
 import numpy as np
 import zunzuncito_amd as zz

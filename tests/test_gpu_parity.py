@@ -116,11 +116,15 @@ def test_golden_zipf_layer(dev):
 @pytest.mark.parametrize("kind,kw,S", [
     ("gemma", dict(), 64), ("gemma", dict(zipf=True, E=64), 37), ("gemma", dict(D=1088, E=64), 16),
     ("lfm", dict(), 48), ("lfm", dict(D=1088), 20), ("maple", dict(E=16), 32),
-    ("ling", dict(), 64), ("ling", dict(D=1088, MI=256), 17)])
+    ("ling", dict(), 64), ("ling", dict(D=1088, MI=256), 17),
+    ("lfm", dict(), 257), ("lfm", dict(D=1088), 137), ("maple", dict(MI=64), 49),
+    ("maple", dict(E=64, D=1088, MI=64), 69), ("ling", dict(), 97), ("ling", dict(D=1088, MI=256), 52)])
 def test_exact_router_logits(dev, kind, kw, S, layer_cache):
-    """At S >= 16 the batched router logits are the reference's own serial chains, bit
-    for bit: gemma's unfused fp32 chain (+ the bias), lfm/maple's double chain and
-    ling's eight double accumulators, each rounded to float as the reference does."""
+    """From 16 tokens (gemma), or from the line between the certified sums and the chains
+    (the other routers; the last six cases lie above it, the five before them below), the
+    batched router logits are the reference's own serial chains, bit for bit: gemma's unfused
+    fp32 chain (+ the bias), lfm/maple's double chain and ling's eight double accumulators,
+    each rounded to float as the reference does. Below it they are the same floats."""
     L = layer_cache(kind, seed=3, **kw)
     say("case", kind, kw, "S", S)
     x = Z.make_input(L, S, 5)
@@ -431,10 +435,10 @@ def test_config4_maple(dev, S, layer_cache):
         m.close()
 
 
-@pytest.mark.parametrize("S", [1, 4, 8, 64])
+@pytest.mark.parametrize("S", [1, 4, 8, 64, 130])
 def test_ling_grouped_router(dev, S, layer_cache):
-    """A13: Ling's grouped router (ling.c:705-789) on the decode (S <= 4), wave-logit
-    (S < 16) and exact-logit (S >= 16) paths: ids exact, weights 1e-4, outputs 1e-3."""
+    """A13: Ling's grouped router (ling.c:705-789) on the decode (S <= 4), wave-logit (S <=
+    96 of its 128 experts) and exact-chain paths: ids exact, weights 1e-4, outputs 1e-3."""
     say("ling grouped S", S)
     L = layer_cache("ling", seed=5)
     x = Z.make_input(L, S, 60 + S)

@@ -272,13 +272,13 @@ def _cancelling_layer(kind, seed):
 
 
 @pytest.mark.parametrize("kind", ["lfm", "maple", "ling"])
-@pytest.mark.parametrize("S", [1, 3, 5, 8, 15])
+@pytest.mark.parametrize("S", [1, 3, 5, 8, 15, 16, 61, 256])
 @pytest.mark.parametrize("cancel", [False, True])
 def test_certified_double_logits(dev, kind, S, cancel):
-    """Below S = 16 the lfm / maple / ling logits come from the wave-parallel sum with
-    the prefix-sum bound of the reference's serial double chain (and a replay where
-    the bound spans a float rounding boundary): they equal the reference's floats bit
-    for bit, and the routing follows."""
+    """Up to 4096 logits of these layers (256 tokens of 16 experts, D = 512; ling 6144) the
+    lfm / maple / ling logits come from the wave-parallel sum with the prefix-sum bound of
+    the reference's serial double chain (and a replay where the bound spans a float rounding
+    boundary): they equal the reference's floats bit for bit, and the routing follows."""
     L = _cancelling_layer(kind, 11 + S) if cancel else small_layer(kind, seed=11 + S)
     x = Z.make_input(L, S, 40 + S)
     if cancel:
