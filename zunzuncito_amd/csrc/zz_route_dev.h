@@ -238,14 +238,14 @@ __device__ __forceinline__ bool zz_exact_sums(const float *w, const float *x, in
     };
     low(tb[l * (ZZ_DPER + 1)]);
     if (!below()) return false;
-#pragma unroll
-    for (int k = 1; k < ZZ_DPER; k++) low(tb[l * (ZZ_DPER + 1) + k]);
-    for (int c0 = 0; c0 + 64 * ZZ_DPER < D; c0 += 64 * ZZ_DPER) {     // the chunks before it, all full
+#pragma unroll 1
+    for (int c0 = 0; c0 < D; c0 += 64 * ZZ_DPER) {
         float wv[ZZ_DPER], xr[ZZ_DPER];
 #pragma unroll
-        for (int j = 0; j < ZZ_DPER; j++) {
-            wv[j] = w[c0 + 64 * j + l];
-            xr[j] = x[c0 + 64 * j + l];
+        for (int j = 0; j < ZZ_DPER; j++) {                  // clamped: the last element again
+            const int i = min(c0 + 64 * j + l, D - 1);
+            wv[j] = w[i];
+            xr[j] = x[i];
         }
 #pragma unroll
         for (int j = 0; j < ZZ_DPER; j++) low((double)wv[j] * (double)xr[j]);
