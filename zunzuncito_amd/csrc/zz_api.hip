@@ -141,12 +141,13 @@ static int grow(float **p, size_t *cap, size_t n) {
     return 1;
 }
 
-// Pinned staging of gpu_matmul, one fixed allocation: calls whose x and y are each up to
-// MM_STAGE floats (1 MiB) have a kernel fetch x from it and another store y into it, in
-// whole lines (stored by the product itself, four rows of a token at a time, a y of 65,536
-// floats crossed the bus in 16-byte pieces and the call took 204 us instead of 165). Whole
-// calls before / now: q4_0 2112 x 2816, 5 tokens 81 / 40 us, 4096 x 2816, 16 tokens 171 / 78.
-// Larger ones, where the bytes and not the two copies' fixed cost count, keep the copies.
+// Pinned staging of gpu_matmul, one fixed allocation until gpu_shutdown: calls whose x and y
+// are each up to MM_STAGE floats (1 MiB) have a kernel fetch x from it and another store y
+// into it, in whole lines (stored by the product itself, four rows of a token at a time, a y
+// of 65,536 floats crossed the bus in 16-byte pieces: 39 us more than the copies). Whole
+// calls, q4_0, with copies / staged: 2112 x 2816, 1 token 44 / 30 us, 5 tokens 41 / 31, 4096
+// x 2816, 16 tokens 64 / 53, 64 tokens, the longest y, 170 / 160. Larger ones, where the
+// bytes and not the two copies' fixed cost count, keep the copies.
 #define MM_STAGE ((size_t)1 << 18)
 static float *g_hx = nullptr, *g_hy = nullptr;
 

@@ -166,12 +166,13 @@ __device__ __forceinline__ void mm_epi(float (&acc)[NT][4], const zz_v4i (&r)[NT
 // activation operand of token tile t, block j (lane l: token 16t + l%16); sx[j] the lane's
 // d_x of block j (mm_epi). The activations are the matrix cores' A rows and the weights
 // their B columns: a lane then holds ONE weight row, whose d_w costs one conversion and one
-// product a block. Bound by VALU issue from three tiles on: with the weights as A rows a
-// lane held four rows (four of each a block) and an output took three operations (d_w * d_x,
+// product a block. The VALU is the busiest unit (63 % of the up kernel's time, 50 % of the
+// down kernel's; the waves wait 36 and 41 % of theirs): with the weights as A rows a lane
+// held four rows (four of each a block) and an output took three operations (d_w * d_x,
 // the integer conversion, the multiply-add) where two do now, 14.0 VALU operations per
-// matrix-core instruction against 10.7 over the whole up kernel. Gemma-4 layer, S = 512,
-// Zipf routing: ffn_up 94.8 -> 86.1 us, ffn_down 61.1 -> 58.2; LFM S = 256 61.0 -> 51.5 and
-// 44.2 -> 38.9; Maple (tq2) S = 512 95.7 -> 86.4 and 59.5 -> 55.6 (HIP events).
+// matrix-core instruction (74 % busy) against 10.8 over the whole up kernel. Gemma-4 layer,
+// S = 512, Zipf routing: ffn_up 94.8 -> 86.1 us, ffn_down 61.1 -> 58.2; LFM S = 256 61.0 ->
+// 51.5 and 44.2 -> 38.9; Maple (tq2) S = 512 95.7 -> 86.4 and 59.5 -> 55.6 (HIP events).
 // DF(j, r): called with block j's int32 results as mm_dot takes them (diagnostics builds
 // store them; the timed build passes a hook that does nothing).
 template <int FMT, int NT, bool FULL, typename XF, typename DF>
@@ -380,7 +381,8 @@ __device__ __forceinline__ void mm_kloop(const uint8_t *E, const ZzTensor &T, in
 // B lane 4b+j = column j, D lane 4b+j, VGPR v = row v). The 4 waves split the K range
 // by chunks (c = w, w+4, ...) and their partial sums meet in LDS. Per 32-weight block
 // a lane spends 12 unpack and 12 epilogue operations for 64 rows x 4 tokens, where
-// the 16x16x32 path spends 4 x 15 for 64 rows x 16 padded tokens. Items of 5-8 tokens
+// the 16x16x32 path spends 4 x 11 for 64 rows x 16 padded tokens (4 x 15 when the limits
+// of 4 and 8 tokens were measured). Items of 5-8 tokens
 // take two token sets (NS = 2, q4_0; q8_0's twice-as-large weight registers would spill):
 // the same weight operand feeds both sets' MFMAs, so a block costs 12 unpack and 24
 // epilogue operations for 64 rows x 8 tokens.
